@@ -453,6 +453,41 @@ int ivakv_index_scatter(void* kv, int64_t s_b, int64_t s_h, int64_t s_s, int64_t
                         int batch, int n_heads, int seq_len, int head_dim,
                         int dtype, hipStream_t stream);
 
+/*
+ * Decoder-layer kernels around the paged attention, for fp16 / bf16 operands (sums in
+ * fp32).  Dense row-major operands, 16-byte aligned.
+ *
+ * ivakv_rms_norm: out = round(round(x / sqrt(mean(x^2) + eps)) * weight) over rows of d
+ * elements (d a multiple of 8 up to 8192); weight may be null.  With a residual, x +
+ * residual (rounded) is normalized instead and also stored to sum.
+ * Replaces: RMSNorm.forward (src/core/norms.py:28-36) and the residual add before it
+ * (src/core/transformer.py:81-151).
+ */
+int ivakv_rms_norm(const void* x, const void* residual, const void* weight, void* sum, void* out,
+                   int64_t rows, int d, float eps, int dtype, hipStream_t stream);
+
+/* out[i] = silu(up[i]) * gate[i], n elements (a multiple of 8).
+ * Replaces: SwiGLU (src/core/ffn.py:21-24,57-60). */
+int ivakv_swiglu(const void* up, const void* gate, void* out, int64_t n, int dtype,
+                 hipStream_t stream);
+
+/*
+ * Linear layers without bias on a few rows: out_i[m][n_i] = x[m][k] . w_i[n_i][k]^T for up
+ * to three matrices (n1, n2 may be 0) in one launch, each streamed once.  m <= 32, k a
+ * multiple of 64, n_i of 16, ldx (the row stride of x, >= k) of 8.
+ *   norm != 0     x is RMS-normalized first, as ivakv_rms_norm does (norm_weight may be
+ *                 null); m <= 16, k <= 2048, epilogue 0 or 2.
+ *   epilogue 1    out0 += residual[m][n0]  (one matrix)
+ *   epilogue 2    out0 = silu(x w1^T) * (x w0^T): w0 the gate, w1 the up projection
+ *                 (n1 == n0, out1 unused)
+ * Replaces: the q / k / v / o projections (src/core/attention.py:46-60,104-110), FFN.forward
+ * (src/core/ffn.py:52-64) and the tied head (src/core/heads.py:31-41) on a decode step's rows.
+ */
+int ivakv_linear_rows(const void* x, int64_t ldx, int m, int k, const void* w0, int n0, void* out0,
+                      const void* w1, int n1, void* out1, const void* w2, int n2, void* out2,
+                      const void* residual, int norm, const void* norm_weight, float eps,
+                      int epilogue, int dtype, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

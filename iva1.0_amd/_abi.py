@@ -179,6 +179,21 @@ SIGNATURES = {
         c_int, c_int, c_int,                   # window, n_sink, dtype
         c_void_p,                              # stream
     ]),
+    "ivakv_rms_norm": (c_int, [
+        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,  # x, residual, weight, sum, out
+        c_int64, c_int, c_float, c_int, c_void_p,  # rows, d, eps, dtype, stream
+    ]),
+    "ivakv_swiglu": (c_int, [
+        c_void_p, c_void_p, c_void_p, c_int64, c_int, c_void_p,  # up, gate, out, n, dtype, stream
+    ]),
+    "ivakv_linear_rows": (c_int, [
+        c_void_p, c_int64, c_int, c_int,       # x, ldx, m, k
+        c_void_p, c_int, c_void_p,             # w0, n0, out0
+        c_void_p, c_int, c_void_p,             # w1, n1, out1
+        c_void_p, c_int, c_void_p,             # w2, n2, out2
+        c_void_p, c_int, c_void_p, c_float,    # residual, norm, norm_weight, eps
+        c_int, c_int, c_void_p,                # epilogue, dtype, stream
+    ]),
     "ivakv_index_gather": (c_int, [
         c_void_p, c_int64, c_int64, c_int64, c_int64,  # kv + strides
         c_void_p, c_int,                             # indices, n_idx

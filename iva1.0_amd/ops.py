@@ -686,6 +686,67 @@ def rope_(x: torch.Tensor, positions: torch.Tensor, theta: float = 10000.0) -> t
     return x
 
 
+# Decoder-layer kernels (ivakv_layer.hip).  The callers in model.py check that the operands
+# are what these take (16-bit, dense, aligned; the sizes below) before they choose them.
+LINEAR_MAX_ROWS = 32       # rows of linear_rows
+LINEAR_NORM_MAX_ROWS = 16  # rows and columns of its fused norm
+LINEAR_NORM_MAX_K = 2048
+NORM_MAX_D = 8192          # columns of rms_norm
+
+
+def rms_norm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float,
+             residual: Optional[torch.Tensor] = None):
+    """RMSNorm over the last dim (src/core/norms.py:28-36); with ``residual`` returns
+    ``(x + residual, norm(x + residual))`` from one pass."""
+    out = torch.empty_like(x)
+    total = torch.empty_like(x) if residual is not None else None
+    d = x.shape[-1]
+    _abi.call("ivakv_rms_norm", x.data_ptr(), residual.data_ptr() if residual is not None else None,
+              weight.data_ptr() if weight is not None else None,
+              total.data_ptr() if total is not None else None, out.data_ptr(), x.numel() // d, d,
+              eps, dtype_code(x.dtype), _stream(x.device))
+    return out if total is None else (total, out)
+
+
+def swiglu(up: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
+    """silu(up) * gate (src/core/ffn.py:21-24,57-60)."""
+    out = torch.empty_like(up)
+    _abi.call("ivakv_swiglu", up.data_ptr(), gate.data_ptr(), out.data_ptr(), up.numel(),
+              dtype_code(up.dtype), _stream(up.device))
+    return out
+
+
+_NO_NORM = (0, None, 0.0)
+
+
+def linear_rows(x: torch.Tensor, weights, norm=None, residual: Optional[torch.Tensor] = None,
+                swiglu_pair: bool = False):
+    """``x @ w.T`` for one to three weight matrices on up to LINEAR_MAX_ROWS rows of ``x`` (all
+    but the last dim), in one launch.  ``norm=(weight, eps)`` RMS-normalizes the rows first;
+    ``residual`` is added to a single product; ``swiglu_pair`` takes ``weights = (gate, up)``
+    and returns ``silu(x @ up.T) * (x @ gate.T)``."""
+    k = x.shape[-1]
+    lead = x.shape[:-1]
+    outs = [torch.empty((*lead, w.shape[0]), dtype=x.dtype, device=x.device)
+            for w in (weights[:1] if swiglu_pair else weights)]
+    args = []
+    for i in range(3):
+        if i < len(weights):
+            args += (weights[i].data_ptr(), weights[i].shape[0],
+                     outs[i].data_ptr() if i < len(outs) else None)
+        else:
+            args += (None, 0, None)
+    if norm is None:
+        norm3 = _NO_NORM
+    else:
+        norm3 = (1, norm[0].data_ptr() if norm[0] is not None else None, norm[1])
+    _abi.call("ivakv_linear_rows", x.data_ptr(), k, x.numel() // k, k, *args,
+              residual.data_ptr() if residual is not None else None, *norm3,
+              2 if swiglu_pair else 1 if residual is not None else 0, dtype_code(x.dtype),
+              _stream(x.device))
+    return outs if len(outs) > 1 else outs[0]
+
+
 def copy_pages(k_pool: torch.Tensor, v_pool: torch.Tensor, src_pages: torch.Tensor,
                dst_pages: torch.Tensor, k_scale: Optional[torch.Tensor] = None,
                v_scale: Optional[torch.Tensor] = None) -> None:

@@ -245,3 +245,34 @@ def test_error_messages_are_per_thread(iva):
     for t in threads:
         t.join()
     assert not bad, bad[:3]
+
+
+def test_layer_kernel_argument_checks(iva):
+    a = iva._abi
+    norm = [FAKE, None, FAKE, None, FAKE]
+    assert call(iva, "ivakv_rms_norm", *norm, 4, 64, 1e-6, a.F32, None) == a.E_DTYPE
+    assert call(iva, "ivakv_rms_norm", *norm, 4, 60, 1e-6, a.F16, None) == a.E_SHAPE
+    assert call(iva, "ivakv_rms_norm", *norm, 4, 8200, 1e-6, a.F16, None) == a.E_SHAPE
+    assert call(iva, "ivakv_rms_norm", FAKE, FAKE, FAKE, None, FAKE, 4, 64, 1e-6, a.F16, None) == a.E_ARG
+    assert call(iva, "ivakv_rms_norm", FAKE + 2, None, None, None, FAKE, 4, 64, 1e-6, a.F16, None) == a.E_ARG
+    assert call(iva, "ivakv_rms_norm", *norm, 0, 64, 1e-6, a.F16, None) == a.OK
+    assert call(iva, "ivakv_swiglu", FAKE, FAKE, FAKE, 12, a.BF16, None) == a.E_SHAPE
+    assert call(iva, "ivakv_swiglu", FAKE, None, FAKE, 16, a.BF16, None) == a.E_ARG
+    assert call(iva, "ivakv_swiglu", None, None, None, 0, a.BF16, None) == a.OK
+
+    def linear(m=4, k=64, n=(16, 16, 16), ldx=None, residual=None, norm=0, epilogue=0, w=FAKE, dtype=a.BF16):
+        mats = []
+        for x in n:
+            mats += [w if x else None, x, FAKE if x else None]
+        return call(iva, "ivakv_linear_rows", FAKE, k if ldx is None else ldx, m, k, *mats, residual, norm,
+                    None, 1e-6, epilogue, dtype, None)
+
+    assert linear(dtype=a.F32) == a.E_DTYPE
+    for bad in (dict(m=33), dict(k=96), dict(n=(16, 8, 16)), dict(ldx=68), dict(norm=1, m=17),
+                dict(norm=1, k=2112), dict(norm=1, epilogue=1, n=(16, 0, 0), residual=FAKE),
+                dict(epilogue=1, residual=FAKE), dict(epilogue=2, n=(16, 32, 0)), dict(epilogue=2)):
+        assert linear(**bad) == a.E_SHAPE, bad
+    for bad in (dict(m=-1), dict(ldx=48), dict(epilogue=3), dict(n=(16, 0, 16)), dict(w=FAKE + 8),
+                dict(epilogue=1, n=(16, 0, 0)), dict(w=None)):
+        assert linear(**bad) == a.E_ARG, bad
+    assert linear(m=0) == a.OK

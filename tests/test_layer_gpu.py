@@ -1,0 +1,126 @@
+"""Decoder-layer kernels (RMSNorm, SwiGLU, few-row linear layers) against float64, and the
+block that fuses them against the same block run module by module.
+
+Bounds: with u = 2^-8 (bf16, 8 significant bits) / 2^-11 (fp16, 11) the largest relative
+error of rounding one value to nearest, an output
+is off by at most u |y| for its own rounding plus what its operands' roundings and the fp32
+sums (k terms, 2^-24 each) carry into it; each test states that sum.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+U = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+DTYPES = [torch.bfloat16, torch.float16]
+
+
+def _randn(shape, seed, dev, dtype, scale=1.0):
+    gen = torch.Generator(device=dev).manual_seed(seed)
+    return (torch.randn(shape, generator=gen, device=dev) * scale).to(dtype)
+
+
+def _norm64(x, w, eps=1e-6):
+    x = x.double()
+    y = x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps)
+    return y if w is None else y * w.double()
+
+
+def _within(got, ref, bound):
+    worst = ((got.double() - ref).abs() - bound).max().item()
+    assert worst <= 0, f"over the bound by {worst}"
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,d", [(1, 8), (3, 512), (5, 520), (16, 1024), (9, 2056), (4, 8192)])
+def test_rms_norm(iva, dev, dtype, rows, d):
+    ops = iva.ops
+    x, r, w = (_randn(s, i, dev, dtype) for i, s in enumerate([(rows, d), (rows, d), (d,)]))
+    # two roundings (y, then y * w) and the fp32 root: 3 u |y|; among fp16's subnormals
+    # (spacing 2^-24) a rounding is off by up to 2^-25 instead, the first one times |w| < 8
+    tiny = 9 * 2.0 ** -25
+    _within(ops.rms_norm(x, w, 1e-6), _norm64(x, w), 3 * U[dtype] * _norm64(x, w).abs() + tiny)
+    _within(ops.rms_norm(x, None, 1e-6), _norm64(x, None), 2 * U[dtype] * _norm64(x, None).abs() + tiny)
+    total, y = ops.rms_norm(x, w, 1e-6, residual=r)
+    assert torch.equal(total, x + r)
+    ref = _norm64(x + r, w)
+    _within(y, ref, 3 * U[dtype] * ref.abs() + tiny)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [8, 2048, 4096 + 8, 100008])
+def test_swiglu(iva, dev, dtype, n):
+    up, gate = _randn(n, 1, dev, dtype, 4.0), _randn(n, 2, dev, dtype)
+    up[:6] = torch.tensor([0.0, -0.0, 300.0, -300.0, float("inf"), float("nan")], dtype=dtype)
+    got, ref = iva.ops.swiglu(up, gate), F.silu(up.double()) * gate.double()
+    assert torch.equal(got[4:6].isnan(), ref[4:6].isnan())
+    ok = ref.isfinite()
+    # one rounding, and exp / reciprocal at 2^-21; 2^-24 absolute covers fp16's subnormals
+    _within(got[ok], ref[ok], 1.01 * U[dtype] * ref[ok].abs() + 2.0 ** -24)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k,n", [(64, 16), (320, 48), (1024, 32), (1088, 16), (2048, 64), (4160, 32)])
+@pytest.mark.parametrize("m", [1, 16, 17, 32])
+def test_linear_rows(iva, dev, dtype, m, k, n):
+    ops = iva.ops
+    x = _randn((m, k), 3, dev, dtype)
+    w = [_randn((n * (i + 1), k), 4 + i, dev, dtype, k ** -0.5) for i in range(3)]
+    res, up = _randn((m, n), 8, dev, dtype), _randn((n, k), 9, dev, dtype, k ** -0.5)
+    sums = 2.0 ** -23 * k ** 0.5 * 4  # the fp32 sums of k products of unit variance / k
+
+    def check(got, ref, extra=0.0):
+        _within(got, ref, 1.01 * U[dtype] * ref.abs() + sums + extra)
+
+    for got, wi in zip(ops.linear_rows(x, w), w):
+        check(got, x.double() @ wi.double().t())
+    check(ops.linear_rows(x, w[:1], residual=res), x.double() @ w[0].double().t() + res.double())
+    ug = x.double() @ up.double().t(), x.double() @ w[0].double().t()
+    check(ops.linear_rows(x, [w[0], up], swiglu_pair=True), F.silu(ug[0]) * ug[1],
+          2 * sums * (1 + ug[0].abs() + ug[1].abs()))
+    if m <= ops.LINEAR_NORM_MAX_ROWS and k <= ops.LINEAR_NORM_MAX_K:
+        nw = _randn(k, 10, dev, dtype)
+        y = ops.rms_norm(x, nw, 1e-6)  # the fused norm rounds as the kernel alone does
+        for got, alone in zip(ops.linear_rows(x, w, norm=(nw, 1e-6)), ops.linear_rows(y, w)):
+            assert torch.equal(got, alone)
+        assert torch.equal(ops.linear_rows(x, [w[0], up], norm=(nw, 1e-6), swiglu_pair=True),
+                           ops.linear_rows(y, [w[0], up], swiglu_pair=True))
+
+
+def test_linear_rows_many_tiles(iva, dev):
+    """More column tiles than workgroups: each takes several, an odd number of them."""
+    n, k = 16 * (2 * 1024 + 333), 1024
+    x, w = _randn((16, k), 1, dev, torch.bfloat16), _randn((n, k), 2, dev, torch.bfloat16, k ** -0.5)
+    ref = x.double() @ w.double().t()
+    _within(iva.ops.linear_rows(x, (w,)), ref, 1.01 * U[torch.bfloat16] * ref.abs() + 2.0 ** -16)
+
+
+@pytest.mark.parametrize("d_model,heads,kv", [(256, 4, 2), (1024, 16, 16), (2560, 10, 10)])
+@pytest.mark.parametrize("batch,tokens", [(1, 2), (16, 1), (2, 12), (3, 40)])
+def test_fused_block_matches_modules(iva, dev, d_model, heads, kv, batch, tokens):
+    """The fused block and the same block with a hook on a submodule, which makes it run
+    module by module (and the hook fire)."""
+    M = iva.model
+    cfg = M.TransformerConfig(d_model=d_model, n_heads=heads, n_kv_heads=kv, n_layers=1, vocab_size=64,
+                              seq_len=128, dropout=0.1, attn_impl="hip_paged")
+    torch.manual_seed(5)
+    block = M.Transformer(cfg).to(dev, torch.bfloat16).eval().blocks[0]
+    x = _randn((batch, tokens, d_model), 6, dev, torch.bfloat16)
+    with torch.no_grad():
+        fused = block(x)[0]
+        calls = []
+        hooks = [m.register_forward_hook(lambda mod, i, o: calls.append(type(mod).__name__))
+                 for m in (block.attention.o_proj, block.ffn.down_proj, block.norm2)]
+        alone = block(x)[0]
+        for h in hooks:
+            h.remove()
+        with torch.enable_grad():
+            grad = block.norm1(x.requires_grad_())
+        assert grad.requires_grad
+    assert sorted(calls) == ["Linear", "Linear", "RMSNorm"]
+    # both round every intermediate once or twice to bf16, six in a row
+    err = (fused.double() - alone.double()).norm() / alone.double().norm()
+    assert err <= 6 * U[torch.bfloat16], err
