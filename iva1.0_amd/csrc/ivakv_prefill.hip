@@ -137,7 +137,9 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   constexpr int NB = D / 16;      // 16-dim blocks
   constexpr int NR = S::NR;
   constexpr int64_t kTile = (int64_t)D * kBS;
-  extern __shared__ Chunk16 lds[];  // 2 x [K_A | K_B | V_A | V_B], global tile layout
+  extern __shared__ Chunk16 lds[];  // kBufs x [K_A | K_B | V_A | V_B], global tile layout
+  __shared__ int s_bad[S::kWaves];
+  bool any_bad = false;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, ln = lane & 15, lq = lane >> 4;
@@ -195,120 +197,104 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
     l_run[rb] = 0.f;
   }
 
-  // Pair staging, HBM -> registers -> LDS.  An LDS buffer holds
-  //   [K_A | K_B]  the two K tiles in the pools' layout (16-byte chunks), and
-  //   V pair       row d (32 keys) = granules A0 B0 A1 B1 A2 B2 A3 B3, granule
-  //                Pg = keys 4g..4g+3 of page P (4 elements),
-  // so a lane's PV operand (granule lq of page A and of page B for dim d) is one
-  // contiguous 2-granule read and a wave's V reads are conflict-free.  Thread
-  // tid moves 16-byte LDS chunks tid + T*c of each part.  Pages past n_eff are
-  // clamped to the last one (masked later); invalid ids read page 0.
+  // Pair staging, HBM -> registers -> LDS.  An LDS buffer holds the four tiles [K_A | K_B |
+  // V_A | V_B] in the pools' layout, copied in 16-byte chunks: chunk c of the buffer is
+  // chunk c % kPageChunks of tile c / kPageChunks, moved by thread c % kThreads.  Which 32
+  // keys a lane holds follows from what makes V's rows readable in that layout: lane (ln, lq)
+  // reads 16 bytes (32 for fp32) of a V row, the 8 keys 8 (lq & 1) .. + 7 of page lq >> 1,
+  // so it has to hold those 8 keys' scores, and the two QK products take K's rows in that
+  // order (row i of the first is key 8 ((i >> 2) & 1) + (i & 3) of page i >> 3, of the second
+  // the key 4 above).  K_B's rows are stored with their index ^ 4, so one read's 16 rows lie
+  // in 16 different 16-byte columns of the banks.
+  //
+  // A thread's chunks come from page A or B by its index (two pages' tiles at most as many
+  // chunks as threads) or by the chunk's number, so it fetches one page id per pair, or
+  // two: with vector loads two pairs ahead (no scalar-memory wait inside a step: the scalar
+  // and LDS counters are shared), in the slot of the pair's parity.  Pages past v_end are
+  // the last one (masked later); an invalid id reads page 0, and its V rows are zeroed.
   constexpr int kPageChunks = S::kPageElems * (int)sizeof(E) / 16;
-  constexpr int kGran = 4 * (int)sizeof(E);  // bytes of one V granule
-  constexpr int kKPer = (2 * kPageChunks + S::kThreads - 1) / S::kThreads;
-  constexpr int kVPer = kKPer;               // the V pair has as many 16-byte chunks
+  constexpr bool kOneId = S::kThreads >= 2 * kPageChunks;
+  constexpr int kIds = kOneId ? 1 : 2;
+  constexpr int kChunks = 4 * kPageChunks / S::kThreads;  // per thread and pair
+  static_assert(4 * kPageChunks % S::kThreads == 0 &&
+                (kOneId || kPageChunks % S::kThreads == 0), "chunks of a pair per thread");
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  u32x4 stK[S::kStages][kKPer], stV[S::kStages][kVPer];  // vector types: kept in registers
-  // Page ids.  Lanes fetch the block-table entries of a pair two loads ahead
-  // with vector loads (no scalar-memory wait inside a step: the scalar and LDS
-  // counters are shared), into the slot of the pair's parity; load() moves them
-  // to scalar registers and records each page's validity (id in range, page
-  // inside the walk) in okmask, bits 2 (pair % 16) and + 1, which the pair's
-  // step reads.  Pages past n_eff are the last one (masked later); invalid ids
-  // read page 0.
+  u32x4 st[S::kStages][kFp8 ? 1 : kChunks];  // vector types: kept in registers
+  const int own_pg = (tid / kPageChunks) & 1;  // kOneId: the page of this thread's chunks
   auto lpage = [&](int v) IVAKV_INLINE -> int { return logical_page(w, v < v_end ? v : v_end - 1); };
   const int32_t* bt_row = bt + (int64_t)b * a.max_blocks;
-  int ids_a[2], ids_b[2];
-  uint32_t okmask = 0;
+  int ids[2][kIds];
   auto fetch_ids = [&](int pair, int par) IVAKV_INLINE {
-    int z = 0;
-    asm volatile("" : "+v"(z));  // a vector-register offset: a vector load
-    ids_a[par] = bt_row[lpage(2 * pair) + z];
-    ids_b[par] = bt_row[lpage(2 * pair + 1) + z];
+    if constexpr (kOneId) {
+      ids[par][0] = bt_row[lpage(2 * pair + own_pg)];
+    } else {
+      int z = 0;
+      asm volatile("" : "+v"(z));  // a vector-register offset: a vector load
+      ids[par][0] = bt_row[lpage(2 * pair) + z];
+      ids[par][kIds - 1] = bt_row[lpage(2 * pair + 1) + z];
+    }
   };
-  auto take_ids = [&](int pair, int par, int64_t& pa, int64_t& pb) IVAKV_INLINE {
-    const int ia = __builtin_amdgcn_readfirstlane(ids_a[par]);
-    const int ib = __builtin_amdgcn_readfirstlane(ids_b[par]);
-    const bool va = ia >= 0 && ia < a.num_pages, vb = ib >= 0 && ib < a.num_pages;
-    const int sh = 2 * (pair & 15);
-    okmask = (okmask & ~(3u << sh)) | ((uint32_t)(va && 2 * pair < n_eff) << sh) |
-             ((uint32_t)(vb && 2 * pair + 1 < n_eff) << (sh + 1));
-    pa = va ? ia : 0;
-    pb = vb ? ib : 0;
+  // The tile of (page id, kv head h), 0 of an invalid id; bad: some lane's id is invalid.
+  auto tile_of = [&](int id, bool& bad) IVAKV_INLINE -> uint64_t {
+    const bool ok = (uint32_t)id < (uint32_t)a.num_pages;
+    bad = __builtin_amdgcn_ballot_w64(!ok) != 0;
+    return (uint64_t)(uint32_t)(ok ? id : 0) * (uint32_t)Hkv + (uint32_t)h;
   };
-  auto pair_ok = [&](int pair) IVAKV_INLINE -> uint32_t { return (okmask >> (2 * (pair & 15))) & 3u; };
+  bool bad[S::kStages][kIds];  // the stage's page has an invalid id (wave-uniform)
+  // First pair whose staged V holds keys at or past L: those rows may hold any bits, and
+  // 0 * NaN would poison the PV accumulator, so they are zeroed as the pair enters LDS.
+  const int v_mask = (L >> 4) >= w.win_first ? w.sink_pages + (L >> 4) - w.win_first
+                                             : min(w.sink_pages, L >> 4);
+  const int vmask_lo = v_end - 1 >= v_mask ? v_mask >> 1 : 0x7fffffff;
+  // Zeroes the elements of V whose keys k0 + i are not attended (page invalid or past L).
+  auto mask_v = [&](u32x4& c, int k0, bool page_bad) IVAKV_INLINE {
+    constexpr int n = 16 / (int)sizeof(E);
+    const int keep = page_bad ? 0 : max(0, min(n, L - k0));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (sizeof(E) == 4) c[i] = i < keep ? c[i] : 0u;
+      else c[i] = 2 * i + 1 < keep ? c[i] : 2 * i < keep ? c[i] & 0xFFFFu : 0u;
+    }
+  };
   auto load_pair = [&](int pair, int set, int par) IVAKV_INLINE {
-    int64_t pa, pb;
-    take_ids(pair, par, pa, pb);
-    const E* kpa = static_cast<const E*>(a.k_pool) + (pa * Hkv + h) * kTile;
-    const E* kpb = static_cast<const E*>(a.k_pool) + (pb * Hkv + h) * kTile;
-    const E* vpa = static_cast<const E*>(a.v_pool) + (pa * Hkv + h) * kTile;
-    const E* vpb = static_cast<const E*>(a.v_pool) + (pb * Hkv + h) * kTile;
+    if constexpr (!kFp8) {
+      uint64_t tile[kIds];
 #pragma unroll
-    for (int c = 0; c < kKPer; ++c) {
-      const int idx = min(tid + S::kThreads * c, 2 * kPageChunks - 1);
-      const E* src = idx < kPageChunks ? kpa : kpb;
-      stK[set][c] = *reinterpret_cast<const u32x4*>(src + (idx % kPageChunks) * (16 / (int)sizeof(E)));
-    }
+      for (int i = 0; i < kIds; ++i) tile[i] = tile_of(ids[par][i], bad[set][i]);
 #pragma unroll
-    for (int c = 0; c < kVPer; ++c) {
-      const int v = min(tid + S::kThreads * c, 2 * kPageChunks - 1);
-      if constexpr (kGran == 8) {  // 16-bit: chunk v = row v/4, granule v%4 of A and B
-        const int off = (v >> 2) * kBS + 4 * (v & 3);
-        const u32x2 ga = *reinterpret_cast<const u32x2*>(vpa + off);
-        const u32x2 gb = *reinterpret_cast<const u32x2*>(vpb + off);
-        stV[set][c] = u32x4{ga[0], ga[1], gb[0], gb[1]};
-      } else {  // fp32: chunk v = row v/8, granule (v%8)/2 of page v%2
-        const int off = (v >> 3) * kBS + 4 * ((v & 7) >> 1);
-        stV[set][c] = *reinterpret_cast<const u32x4*>(((v & 1) ? vpb : vpa) + off);
+      for (int c = 0; c < kChunks; ++c) {
+        const int ch = tid + S::kThreads * c;
+        // pool and page of the chunk: by the thread, or (kIds == 2) known at compile time
+        const int pg = kOneId ? 0 : (c * S::kThreads / kPageChunks) & 1;
+        const bool is_v = kChunks == 1 ? ch >= 2 * kPageChunks : 2 * c >= kChunks;
+        const char* pool = static_cast<const char*>(is_v ? a.v_pool : a.k_pool);
+        st[set][c] = *reinterpret_cast<const u32x4*>(pool + tile[pg] * (kTile * sizeof(E)) +
+                                                     16 * (ch % kPageChunks));
       }
+      fetch_ids(pair + 2, par);
     }
-    fetch_ids(pair + 2, par);
-  };
-  // V values of keys no row may see (past the context, on an invalid page) are
-  // zeroed as the pair enters LDS, once for the whole workgroup: 0 * NaN would
-  // poison the PV accumulator.  Only a pair that reaches past the context or
-  // holds an invalid page takes this branch.
-  auto pair_needs_vmask = [&](int pair) IVAKV_INLINE -> bool {
-    return pair_ok(pair) != 3u || lpage(2 * pair + 1) * kBS + kBS > L;
-  };
-  auto v_keys_ok = [&](int pair, int pg, int g, bool (&vis)[4]) IVAKV_INLINE {
-    const bool page_ok = ((pair_ok(pair) >> pg) & 1u) != 0;
-    const int k0 = lpage(2 * pair + pg) * kBS + 4 * g;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) vis[r] = page_ok && k0 + r < L;
   };
   auto store_pair = [&](int buf, int set, int pair) IVAKV_INLINE {
-    u32x4* dk = reinterpret_cast<u32x4*>(lds + buf * (4 * kPageChunks));
-    u32x4* dv = dk + 2 * kPageChunks;
-    if (pair_needs_vmask(pair)) {
+    if constexpr (!kFp8) {
+      u32x4* d = reinterpret_cast<u32x4*>(lds + buf * (4 * kPageChunks));
+      bool any = pair >= vmask_lo;
 #pragma unroll
-      for (int c = 0; c < kVPer; ++c) {
-        const int v = min(tid + S::kThreads * c, 2 * kPageChunks - 1);
-        if constexpr (kGran == 8) {  // granule v%4 of pages A and B
-          bool va[4], vb[4];
-          v_keys_ok(pair, 0, v & 3, va);
-          v_keys_ok(pair, 1, v & 3, vb);
-          Chunk16 ch = __builtin_bit_cast(Chunk16, stV[set][c]);
-          mask_pair16(ch, va, vb);
-          stV[set][c] = __builtin_bit_cast(u32x4, ch);
-        } else {  // granule (v%8)/2 of page v%2
-          bool vis[4];
-          v_keys_ok(pair, v & 1, (v & 7) >> 1, vis);
+      for (int i = 0; i < kIds; ++i) any = any || bad[set][i];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) stV[set][c][r] = vis[r] ? stV[set][c][r] : 0u;
+      for (int c = 0; c < kChunks; ++c) {
+        const int ch = tid + S::kThreads * c;
+        const int pg = kOneId ? own_pg : (c * S::kThreads / kPageChunks) & 1;
+        const bool is_v = kChunks == 1 ? ch >= 2 * kPageChunks : 2 * c >= kChunks;
+        if (any && is_v) {
+          const int in_row = (ch % kPageChunks) % (int)(kBS * sizeof(E) / 16);
+          mask_v(st[set][c], lpage(2 * pair + pg) * kBS + in_row * (16 / (int)sizeof(E)),
+                 bad[set][kOneId ? 0 : pg]);
         }
+        const bool k_b = !is_v && pg == 1;
+        d[k_b ? ch ^ 4 : ch] = st[set][c];
       }
     }
-#pragma unroll
-    for (int c = 0; c < kKPer; ++c)
-      if ((2 * kPageChunks) % S::kThreads == 0 || tid + S::kThreads * c < 2 * kPageChunks)
-        dk[tid + S::kThreads * c] = stK[set][c];
-#pragma unroll
-    for (int c = 0; c < kVPer; ++c)
-      if ((2 * kPageChunks) % S::kThreads == 0 || tid + S::kThreads * c < 2 * kPageChunks)
-        dv[tid + S::kThreads * c] = stV[set][c];
   };
 
   // FP8 staging.  A pair holds 4D 8-byte units of K codes and as many of V codes
@@ -316,8 +302,8 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   // 16(j/32) + 8(j%2) .. +8 of key (j/2)%16, which become the 16-bit pool layout's
   // chunk (2(j/32) + j%2)*16 + key.  V unit j: words 2j, 2j+1 of the tile's FP8
   // order [d%16][key/4][d/16][key%4] (ivakv_internal.h fp8_v_offset), i.e. keys
-  // 4g..4g+3 of dims dl + 16m and dl + 16(m+1), which become granule (g, page) of
-  // those two LDS V rows.
+  // 4g..4g+3 of dims dl + 16m and dl + 16(m+1), which become granule g of those two rows
+  // of the page's LDS V tile.
   constexpr int kUnits = 4 * D;                                  // per pair, K or V
   constexpr int kU8 = kFp8 ? (kUnits + S::kThreads - 1) / S::kThreads : 1;
   constexpr int kNB8 = D / 16;
@@ -326,22 +312,22 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   f32x4 sc8V[S::kStages][kU8];
   auto load_pair8 = [&](int pair, int set, int par) IVAKV_INLINE {
     if constexpr (kFp8) {
-    int64_t pa, pb;
-    take_ids(pair, par, pa, pb);
-    const int64_t tA = pa * Hkv + h, tB = pb * Hkv + h;
-    const uint8_t* k8 = static_cast<const uint8_t*>(a.k_pool);
-    const uint8_t* v8 = static_cast<const uint8_t*>(a.v_pool);
+      uint64_t tile[kIds];
 #pragma unroll
-    for (int c = 0; c < kU8; ++c) {
-      const int u = min(tid + S::kThreads * c, kUnits - 1);
-      const int64_t t = u < 2 * D ? tA : tB;
-      const int j = u % (2 * D);
-      st8K[set][c] = *reinterpret_cast<const u32x2*>(k8 + t * kTile + 8 * j);
-      sc8K[set][c] = a.k_scale[t * kBS + ((j >> 1) & 15)];
-      st8V[set][c] = *reinterpret_cast<const u32x2*>(v8 + t * kTile + 8 * j);
-      sc8V[set][c] = *reinterpret_cast<const f32x4*>(a.v_scale + t * kBS + 4 * (((2 * j) / kNB8) & 3));
-    }
-    fetch_ids(pair + 2, par);
+      for (int i = 0; i < kIds; ++i) tile[i] = tile_of(ids[par][i], bad[set][i]);
+      const uint8_t* k8 = static_cast<const uint8_t*>(a.k_pool);
+      const uint8_t* v8 = static_cast<const uint8_t*>(a.v_pool);
+#pragma unroll
+      for (int c = 0; c < kU8; ++c) {
+        const int u = min(tid + S::kThreads * c, kUnits - 1);
+        const uint64_t t = tile[kOneId ? 0 : (c * S::kThreads / (2 * D)) & 1];
+        const int j = u % (2 * D);
+        st8K[set][c] = *reinterpret_cast<const u32x2*>(k8 + t * kTile + 8 * j);
+        sc8K[set][c] = a.k_scale[t * kBS + ((j >> 1) & 15)];
+        st8V[set][c] = *reinterpret_cast<const u32x2*>(v8 + t * kTile + 8 * j);
+        sc8V[set][c] = *reinterpret_cast<const f32x4*>(a.v_scale + t * kBS + 4 * (((2 * j) / kNB8) & 3));
+      }
+      fetch_ids(pair + 2, par);
     }
   };
   // Four codes (one 32-bit word) times four factors, as four values of E.
@@ -357,17 +343,20 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   auto store_pair8 = [&](int buf, int set, int pair) IVAKV_INLINE {
     if constexpr (kFp8) {
     u32x4* dk = reinterpret_cast<u32x4*>(lds + buf * (4 * kPageChunks));
-    u32x2* dv = reinterpret_cast<u32x2*>(dk + 2 * kPageChunks);  // V rows of 8 granules
+    u32x2* dv = reinterpret_cast<u32x2*>(dk + 2 * kPageChunks);  // V rows of 4 granules
+    bool any = pair >= vmask_lo;
+#pragma unroll
+    for (int i = 0; i < kIds; ++i) any = any || bad[set][i];
 #pragma unroll
     for (int c = 0; c < kU8; ++c) {
       if (kUnits % S::kThreads != 0 && tid + S::kThreads * c >= kUnits) continue;
       const int u = tid + S::kThreads * c;
-      const int pg = u < 2 * D ? 0 : 1, j = u % (2 * D);
+      const int pg = kOneId ? own_pg : (c * S::kThreads / (2 * D)) & 1, j = u % (2 * D);
       // K: one key's 8 dims, one 16-byte LDS chunk
       const float ik = __builtin_amdgcn_rcpf(sc8K[set][c]);
       const u32x2 k0 = dequant4(st8K[set][c][0], ik, ik, ik, ik);
       const u32x2 k1 = dequant4(st8K[set][c][1], ik, ik, ik, ik);
-      const int key = (j >> 1) & 15, ch = (2 * (j >> 5) + (j & 1)) * 16 + key;
+      const int key = (j >> 1) & 15, ch = (2 * (j >> 5) + (j & 1)) * 16 + (pg ? key ^ 4 : key);
       dk[pg * kPageChunks + ch] = u32x4{k0[0], k0[1], k1[0], k1[1]};
       // V: keys 4g..4g+3 of two dims, one 8-byte granule in each of two rows
       const f32x4 sv = sc8V[set][c];
@@ -377,18 +366,16 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
       u32x2 vv[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e) vv[e] = dequant4(st8V[set][c][e], i0, i1, i2, i3);
-      if (pair_needs_vmask(pair)) {
-        bool vis[4];
-        v_keys_ok(pair, pg, g, vis);
+      if (any) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          Chunk8 h = __builtin_bit_cast(Chunk8, vv[e]);
-          mask_rows16(h, vis);
-          vv[e] = __builtin_bit_cast(u32x2, h);
+          u32x4 h4{vv[e][0], vv[e][1], 0u, 0u};
+          mask_v(h4, lpage(2 * pair + pg) * kBS + 4 * g, bad[set][kOneId ? 0 : pg]);
+          vv[e] = u32x2{h4[0], h4[1]};
         }
       }
 #pragma unroll
-      for (int e = 0; e < 2; ++e) dv[(dl + 16 * (m + e)) * 8 + 2 * g + pg] = vv[e];
+      for (int e = 0; e < 2; ++e) dv[pg * (2 * kPageChunks) + (dl + 16 * (m + e)) * 4 + g] = vv[e];
     }
     }
   };
@@ -405,24 +392,32 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   struct PairS {
     f32x4 sa[NR], sb[NR];
   };
-  // A pair past the walk or entirely after every row of the wave is skipped.
-  auto pair_live = [&](int pair) IVAKV_INLINE -> bool {
-    return pair < n_pairs && lpage(2 * pair) * kBS <= wave_p_hi;
-  };
+  // A pair past the walk or entirely after every row of the wave is skipped: the wave's
+  // rows see pages up to the one of wave_p_hi.
+  const int p_seen = wave_p_hi >> 4;
+  const int live_end =
+      wave_p_hi < 0 ? 0
+                    : min(n_pairs, ((p_seen >= w.win_first ? w.sink_pages + p_seen - w.win_first + 1
+                                                           : min(w.sink_pages, p_seen + 1)) + 1) >> 1);
+  auto pair_live = [&](int pair) IVAKV_INLINE -> bool { return pair < live_end; };
+  // This lane's K row of the first QK product (of the second: index ^ 4), and its V bytes.
+  const int k_row = 8 * ((ln >> 2) & 1) + (ln & 3), k_pg = ln >> 3;
+  const int k_off1 = (k_pg * kPageChunks + lq * kBS + (k_row ^ (4 * k_pg))) * 16, k_off2 = k_off1 ^ 64;
+  const int v_off = (2 * kPageChunks + (lq >> 1) * kPageChunks) * 16 +
+                    (ln * kBS + 8 * (lq & 1)) * (int)sizeof(E);
   auto read_k = [&](int buf, Chunk16 (&ka)[KLD], Chunk16 (&kb)[KLD]) IVAKV_INLINE {
-    const E* kA = reinterpret_cast<const E*>(lds + buf * (4 * kPageChunks));
-    const E* kB = kA + S::kPageElems;
+    const char* base = reinterpret_cast<const char*>(lds + buf * (4 * kPageChunks));
 #pragma unroll
     for (int j = 0; j < KLD; ++j) {
-      ka[j] = *reinterpret_cast<const Chunk16*>(kA + ((4 * j + lq) * kBS + ln) * X);
-      kb[j] = *reinterpret_cast<const Chunk16*>(kB + ((4 * j + lq) * kBS + ln) * X);
+      ka[j] = *reinterpret_cast<const Chunk16*>(base + k_off1 + 64 * kBS * j);
+      kb[j] = *reinterpret_cast<const Chunk16*>(base + k_off2 + 64 * kBS * j);
     }
   };
   using VPair = typename Tr::VPair;
   auto read_v = [&](int buf, VPair (&vp)[NB]) IVAKV_INLINE {
-    const char* vP = reinterpret_cast<const char*>(lds + buf * (4 * kPageChunks) + 2 * kPageChunks);
+    const char* base = reinterpret_cast<const char*>(lds + buf * (4 * kPageChunks)) + v_off;
 #pragma unroll
-    for (int m = 0; m < NB; ++m) vp[m] = Tr::read_vpair(vP + (16 * m + ln) * (8 * kGran) + lq * (2 * kGran));
+    for (int m = 0; m < NB; ++m) vp[m] = Tr::read_vpair(base + 16 * kBS * (int)sizeof(E) * m);
   };
   auto qk_mfma = [&](const Chunk16 (&ka)[KLD], const Chunk16 (&kb)[KLD], PairS& sc) IVAKV_INLINE {
 #pragma unroll
@@ -490,17 +485,24 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   // place: keys a row must not see (after its position, outside its window and
   // not a sink, past the context, on an invalid page) get score -inf.
   auto mask_scores = [&](int pair, PairS& sc) IVAKV_INLINE {
-    const uint32_t ok = pair_ok(pair);
-    const bool oka = (ok & 1u) != 0, okb = (ok & 2u) != 0;
-    const int ka0 = lpage(2 * pair) * kBS + 4 * lq, kb0 = lpage(2 * pair + 1) * kBS + 4 * lq;
+    const int v = 2 * pair + (lq >> 1);  // this lane's page
+    bool ok = v < n_eff;
+    const int lp = lpage(v);
+    if (any_bad) {  // uniform: some page of the walk is invalid
+      const int id = bt_row[lp];
+      ok = ok && id >= 0 && id < a.num_pages;
+    }
+    const int k0 = lp * kBS + 8 * (lq & 1);
 #pragma unroll
     for (int rb = 0; rb < NR; ++rb) {
-      const int qp = qpos[rb];
+      const int qp = ok ? qpos[rb] : -1;
+      // the keys the row sees: up to qp, from lo on or below the sinks
+      const int lo = a.window > 0 ? qp - a.window + 1 : 0, sinks = a.window > 0 ? a.n_sink : 0;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int ka_ = ka0 + r, kb_ = kb0 + r;
-        const bool visa = oka && ka_ <= qp && (a.window <= 0 || ka_ > qp - a.window || ka_ < a.n_sink);
-        const bool visb = okb && kb_ <= qp && (a.window <= 0 || kb_ > qp - a.window || kb_ < a.n_sink);
+        const int ka_ = k0 + r, kb_ = k0 + 4 + r;
+        const bool visa = ka_ <= qp && (ka_ >= lo || ka_ < sinks);
+        const bool visb = kb_ <= qp && (kb_ >= lo || kb_ < sinks);
         sc.sa[rb][r] = visa ? sc.sa[rb][r] : kNegInf;
         sc.sb[rb][r] = visb ? sc.sb[rb][r] : kNegInf;
       }
@@ -510,13 +512,15 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   // the wave: both pages valid and inside the walk, every key at or before the
   // wave's first row position and inside the window of its last row.  (Rows past
   // the chunk's end read row 0's query, so their scores stay finite; they are
-  // never stored.)
+  // never stored.)  Past the sink pages logical pages are consecutive, so these are the
+  // pairs [int_lo, int_hi); pairs with sink pages before a window are masked.
   const int wave_pos_lo = first_pos + r_w / G;  // may be negative: then no pair is
-  auto interior = [&](int pair) IVAKV_INLINE -> bool {
-    return wave_pos_lo >= 0 && pair_ok(pair) == 3u &&
-           lpage(2 * pair + 1) * kBS + kBS - 1 <= wave_pos_lo &&
-           (a.window <= 0 || lpage(2 * pair) * kBS > wave_p_hi - a.window);
-  };
+  const int d_lp = w.win_first - w.sink_pages;
+  int int_lo = (w.sink_pages + 1) >> 1, int_hi = 0;
+  if (a.window > 0 && wave_p_hi - a.window >= 0)
+    int_lo = max(int_lo, (((wave_p_hi - a.window) >> 4) + 1 - d_lp + 1) >> 1);
+  if (wave_pos_lo >= 0) int_hi = min(n_eff >> 1, (((wave_pos_lo + 1) >> 4) - d_lp) >> 1);
+  auto interior = [&](int pair) IVAKV_INLINE -> bool { return pair >= int_lo && pair < int_hi; };
   // Softmax and PV of a pair, with the next pair's QK (with_next): one test for
   // any row max growing (rare), then one block with no branch: the next pair's K
   // reads and QK MFMAs, this pair's V reads, exponentials and PV MFMAs.
@@ -557,12 +561,31 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
     softmax_pv(std::false_type{}, buf, sc, buf, sc);
   };
 
+  // Whether any page of this call's pairs has an invalid id (then no pair is interior, and
+  // the masks read the ids): each thread looks at a part of the table row, and the waves'
+  // findings meet at the first barrier.
+  auto scan_ids = [&]() IVAKV_INLINE {
+    bool found = false;
+    for (int v = 2 * p0 + tid; v < v_end; v += S::kThreads)
+      found = found || (uint32_t)bt_row[lpage(v)] >= (uint32_t)a.num_pages;
+    if (lane == 0) s_bad[wave] = 0;
+    if (found) s_bad[wave] = 1;
+  };
+  auto take_scan = [&]() IVAKV_INLINE {
+    int found = 0;
+#pragma unroll
+    for (int i = 0; i < S::kWaves; ++i) found |= s_bad[i];
+    any_bad = uni(found) != 0;
+    if (any_bad) int_hi = 0;
+  };
+
   // Ring: pair i is in LDS buffer i % 2 while pair i + 1 travels from HBM / L2
   // into the staging registers; one barrier per pair.  Page ids are fetched two
   // loads ahead, in the slot of the pair's parity.
   if (n_pairs > p0) {
     fetch_ids(p0, 0);
     fetch_ids(p0 + 1, 1);
+    scan_ids();
     if constexpr (S::kStages == 2) {
       // Software pipeline over eight LDS buffers (pair p in buffer p & 7) and two
       // stage sets (pair p in set p % 2), two steps and one barrier per
@@ -584,6 +607,7 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
       store((p0 + 2) & 7, 0, p0 + 2);
       load(p0 + 4, 0, 0);
       __syncthreads();
+      take_scan();
       if (pair_live(p0)) qk_pair(p0 & 7, s0);
       for (int i = p0; i < n_pairs; i += 2) {
         store((i + 3) & 7, 1, i + 3);
@@ -600,6 +624,7 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
       load(p0, 0, 0);
       store(0, 0, p0);
       __syncthreads();
+      take_scan();
       for (int i = p0; i < n_pairs; i += 2) {
         load(i + 1, 0, 1);
         compute(0, i);
