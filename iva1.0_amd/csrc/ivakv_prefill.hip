@@ -222,6 +222,11 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   u32x4 st[S::kStages][kFp8 ? 1 : kChunks];  // vector types: kept in registers
   const int own_pg = (tid / kPageChunks) & 1;  // kOneId: the page of this thread's chunks
+  // Chunks of one page (all kv heads), and this thread's first chunk of kv head h's tiles.
+  const uint32_t page_chunks = (uint32_t)Hkv * (uint32_t)kPageChunks;
+  const uint64_t first_chunk = (uint64_t)(uint32_t)h * kPageChunks + tid % kPageChunks;
+  const u32x4* tile_k = static_cast<const u32x4*>(a.k_pool) + first_chunk;
+  const u32x4* tile_v = static_cast<const u32x4*>(a.v_pool) + first_chunk;
   auto lpage = [&](int v) IVAKV_INLINE -> int { return logical_page(w, v < v_end ? v : v_end - 1); };
   const int32_t* bt_row = bt + (int64_t)b * a.max_blocks;
   int ids[2][kIds];
@@ -235,18 +240,18 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
       ids[par][kIds - 1] = bt_row[lpage(2 * pair + 1) + z];
     }
   };
-  // The tile of (page id, kv head h), 0 of an invalid id; bad: some lane's id is invalid.
-  auto tile_of = [&](int id, bool& bad) IVAKV_INLINE -> uint64_t {
-    const bool ok = (uint32_t)id < (uint32_t)a.num_pages;
-    bad = __builtin_amdgcn_ballot_w64(!ok) != 0;
-    return (uint64_t)(uint32_t)(ok ? id : 0) * (uint32_t)Hkv + (uint32_t)h;
-  };
-  bool bad[S::kStages][kIds];  // the stage's page has an invalid id (wave-uniform)
-  // First pair whose staged V holds keys at or past L: those rows may hold any bits, and
-  // 0 * NaN would poison the PV accumulator, so they are zeroed as the pair enters LDS.
+  auto id_ok = [&](int id) IVAKV_INLINE -> bool { return (uint32_t)id < (uint32_t)a.num_pages; };
+  int st_id[S::kStages][kIds];  // page ids of the staged pairs
+  // (two ids per thread, where the vector registers are full, go to scalar ones)
+  auto staged_id = [&](int id) IVAKV_INLINE -> int { return kOneId ? id : uni(id); };
+  // First pair whose staged V may hold rows no query sees: keys at or past L, or, when a
+  // page of the walk is invalid, any (so until the scan of the ids is in).  Such rows may
+  // hold any bits, and 0 * NaN would poison the PV accumulator: they are zeroed as the pair
+  // enters LDS.
   const int v_mask = (L >> 4) >= w.win_first ? w.sink_pages + (L >> 4) - w.win_first
                                              : min(w.sink_pages, L >> 4);
-  const int vmask_lo = v_end - 1 >= v_mask ? v_mask >> 1 : 0x7fffffff;
+  const int vmask_tail = v_end - 1 >= v_mask ? v_mask >> 1 : 0x7fffffff;
+  int vmask_lo = 0;
   // Zeroes the elements of V whose keys k0 + i are not attended (page invalid or past L).
   auto mask_v = [&](u32x4& c, int k0, bool page_bad) IVAKV_INLINE {
     constexpr int n = 16 / (int)sizeof(E);
@@ -259,18 +264,20 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   };
   auto load_pair = [&](int pair, int set, int par) IVAKV_INLINE {
     if constexpr (!kFp8) {
-      uint64_t tile[kIds];
+      uint64_t page[kIds];  // the pages' first chunks (of the pools, in 16-byte chunks)
 #pragma unroll
-      for (int i = 0; i < kIds; ++i) tile[i] = tile_of(ids[par][i], bad[set][i]);
+      for (int i = 0; i < kIds; ++i) {
+        const int id = st_id[set][i] = staged_id(ids[par][i]);
+        page[i] = (uint64_t)(uint32_t)(id_ok(id) ? id : 0) * page_chunks;
+      }
 #pragma unroll
       for (int c = 0; c < kChunks; ++c) {
         const int ch = tid + S::kThreads * c;
         // pool and page of the chunk: by the thread, or (kIds == 2) known at compile time
         const int pg = kOneId ? 0 : (c * S::kThreads / kPageChunks) & 1;
         const bool is_v = kChunks == 1 ? ch >= 2 * kPageChunks : 2 * c >= kChunks;
-        const char* pool = static_cast<const char*>(is_v ? a.v_pool : a.k_pool);
-        st[set][c] = *reinterpret_cast<const u32x4*>(pool + tile[pg] * (kTile * sizeof(E)) +
-                                                     16 * (ch % kPageChunks));
+        const u32x4* tile = (is_v ? tile_v : tile_k) + (kChunks <= 2 ? 0 : S::kThreads * c % kPageChunks);
+        st[set][c] = tile[page[pg]];
       }
       fetch_ids(pair + 2, par);
     }
@@ -278,9 +285,7 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   auto store_pair = [&](int buf, int set, int pair) IVAKV_INLINE {
     if constexpr (!kFp8) {
       u32x4* d = reinterpret_cast<u32x4*>(lds + buf * (4 * kPageChunks));
-      bool any = pair >= vmask_lo;
-#pragma unroll
-      for (int i = 0; i < kIds; ++i) any = any || bad[set][i];
+      const bool any = pair >= vmask_lo;
 #pragma unroll
       for (int c = 0; c < kChunks; ++c) {
         const int ch = tid + S::kThreads * c;
@@ -289,7 +294,7 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
         if (any && is_v) {
           const int in_row = (ch % kPageChunks) % (int)(kBS * sizeof(E) / 16);
           mask_v(st[set][c], lpage(2 * pair + pg) * kBS + in_row * (16 / (int)sizeof(E)),
-                 bad[set][kOneId ? 0 : pg]);
+                 !id_ok(st_id[set][kOneId ? 0 : pg]));
         }
         const bool k_b = !is_v && pg == 1;
         d[k_b ? ch ^ 4 : ch] = st[set][c];
@@ -314,7 +319,10 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
     if constexpr (kFp8) {
       uint64_t tile[kIds];
 #pragma unroll
-      for (int i = 0; i < kIds; ++i) tile[i] = tile_of(ids[par][i], bad[set][i]);
+      for (int i = 0; i < kIds; ++i) {
+        const int id = st_id[set][i] = staged_id(ids[par][i]);
+        tile[i] = (uint64_t)(uint32_t)(id_ok(id) ? id : 0) * (uint32_t)Hkv + (uint32_t)h;
+      }
       const uint8_t* k8 = static_cast<const uint8_t*>(a.k_pool);
       const uint8_t* v8 = static_cast<const uint8_t*>(a.v_pool);
 #pragma unroll
@@ -344,9 +352,7 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
     if constexpr (kFp8) {
     u32x4* dk = reinterpret_cast<u32x4*>(lds + buf * (4 * kPageChunks));
     u32x2* dv = reinterpret_cast<u32x2*>(dk + 2 * kPageChunks);  // V rows of 4 granules
-    bool any = pair >= vmask_lo;
-#pragma unroll
-    for (int i = 0; i < kIds; ++i) any = any || bad[set][i];
+    const bool any = pair >= vmask_lo;
 #pragma unroll
     for (int c = 0; c < kU8; ++c) {
       if (kUnits % S::kThreads != 0 && tid + S::kThreads * c >= kUnits) continue;
@@ -370,7 +376,7 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           u32x4 h4{vv[e][0], vv[e][1], 0u, 0u};
-          mask_v(h4, lpage(2 * pair + pg) * kBS + 4 * g, bad[set][kOneId ? 0 : pg]);
+          mask_v(h4, lpage(2 * pair + pg) * kBS + 4 * g, !id_ok(st_id[set][kOneId ? 0 : pg]));
           vv[e] = u32x2{h4[0], h4[1]};
         }
       }
@@ -444,20 +450,31 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
       sl[4 + r] = sc.sb[rb][r];
     }
   };
-  auto scaled_max = [&](const float (&sl)[8]) IVAKV_INLINE -> float {
-    float lmx = sl[0];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) lmx = fmaxf(lmx, sl[i]);
-    return lmx * c_log2;
-  };
   // Lazy rescaling: the reference max m_run of a row (log2 units) only moves
   // (with a cross-lane max and a rescale of acc and l) when a scaled score exceeds
   // it by more than kLazyMax; otherwise p = exp2(s*c - m_run) <= 2^kLazyMax and
-  // the final O = acc / l is unchanged.
-  auto grows = [&](int rb, float lmx) IVAKV_INLINE -> bool { return lmx > m_run[rb] + kLazyMax; };
-  auto rescale = [&](int rb, float lmx) IVAKV_INLINE {
-    if (__builtin_amdgcn_ballot_w64(grows(rb, lmx)) != 0) {
-      float mx = fmaxf(lmx, __shfl_xor(lmx, 16));
+  // the final O = acc / l is unchanged.  grow_at is that bound in raw scores, (m_run +
+  // kLazyMax) / c, and neg_m what the exponent adds, -m_run (0 while no key was seen).
+  float grow_at[NR], neg_m[NR];
+#pragma unroll
+  for (int rb = 0; rb < NR; ++rb) {
+    grow_at[rb] = kNegInf;
+    neg_m[rb] = 0.f;
+  }
+  const float inv_c = 1.f / c_log2;
+  auto grows = [&](int rb, const float (&sl)[8]) IVAKV_INLINE -> bool {
+    float mx = fmaxf(fmaxf(grow_at[rb], sl[0]), sl[1]);
+#pragma unroll
+    for (int i = 2; i < 8; i += 2) mx = fmaxf(fmaxf(mx, sl[i]), sl[i + 1]);
+    return mx > grow_at[rb];
+  };
+  auto rescale = [&](int rb, const float (&sl)[8]) IVAKV_INLINE {
+    if (__builtin_amdgcn_ballot_w64(grows(rb, sl)) != 0) {
+      float mx = sl[0];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) mx = fmaxf(mx, sl[i]);
+      mx *= c_log2;
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
       mx = fmaxf(mx, __shfl_xor(mx, 32));
       const float m_new = fmaxf(m_run[rb], mx);
       const float alpha = m_new == kNegInf ? 1.f : exp2_fast(m_run[rb] - m_new);
@@ -465,16 +482,17 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
 #pragma unroll
       for (int m = 0; m < NB; ++m) acc[rb][m] *= alpha;
       m_run[rb] = m_new;
+      grow_at[rb] = (m_new + kLazyMax) * inv_c;
+      neg_m[rb] = m_new == kNegInf ? 0.f : -m_new;
     }
   };
   // p = exp2(s*c - m_run) of the lane's 8 scores, their sum into l, PV.
   auto exp_pv = [&](int rb, const float (&sl)[8], const VPair (&vp)[NB]) IVAKV_INLINE {
-    const float m_use = m_run[rb] == kNegInf ? 0.f : m_run[rb];
     float pa[4], pb[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      pa[r] = exp2_fast(__builtin_fmaf(sl[r], c_log2, -m_use));
-      pb[r] = exp2_fast(__builtin_fmaf(sl[4 + r], c_log2, -m_use));
+      pa[r] = exp2_fast(__builtin_fmaf(sl[r], c_log2, neg_m[rb]));
+      pb[r] = exp2_fast(__builtin_fmaf(sl[4 + r], c_log2, neg_m[rb]));
     }
     l_run[rb] += ((pa[0] + pa[1]) + (pa[2] + pa[3])) + ((pb[0] + pb[1]) + (pb[2] + pb[3]));
     const typename Tr::PP8 p8 = Tr::pack_pp8(pa, pb);
@@ -526,17 +544,16 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
   // reads and QK MFMAs, this pair's V reads, exponentials and PV MFMAs.
   auto softmax_pv = [&](auto with_next, int bn, PairS& sn, int bc, const PairS& sc) IVAKV_INLINE {
     constexpr bool kNext = decltype(with_next)::value;
-    float sl[NR][8], lmx[NR];
+    float sl[NR][8];
     bool any = false;
 #pragma unroll
     for (int rb = 0; rb < NR; ++rb) {
       lane_scores(sc, rb, sl[rb]);
-      lmx[rb] = scaled_max(sl[rb]);
-      any = any || grows(rb, lmx[rb]);
+      any = any || grows(rb, sl[rb]);
     }
     if (__builtin_amdgcn_ballot_w64(any) != 0) {
 #pragma unroll
-      for (int rb = 0; rb < NR; ++rb) rescale(rb, lmx[rb]);
+      for (int rb = 0; rb < NR; ++rb) rescale(rb, sl[rb]);
     }
     if constexpr (kNext) qk_pair(bn, sn);
     VPair vp[NB];
@@ -577,6 +594,7 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
     for (int i = 0; i < S::kWaves; ++i) found |= s_bad[i];
     any_bad = uni(found) != 0;
     if (any_bad) int_hi = 0;
+    else vmask_lo = vmask_tail;
   };
 
   // Ring: pair i is in LDS buffer i % 2 while pair i + 1 travels from HBM / L2
