@@ -454,6 +454,15 @@ int ivakv_index_scatter(void* kv, int64_t s_b, int64_t s_h, int64_t s_s, int64_t
                         int dtype, hipStream_t stream);
 
 /*
+ * Slots of the last n positions of each sequence: slots[b * n + t] = the slot of position
+ * context_lens[b] - n + t (int32; -1 where the position is negative, past the table or on
+ * no page), the slot_mapping of an append of n new tokens per sequence.
+ * Replaces: the start_pos arithmetic of KVCache.update (src/core/rope_kv.py:98-110).
+ */
+int ivakv_chunk_slots(const int32_t* block_tables, const int32_t* context_lens, int batch, int n,
+                      int max_blocks, int block_size, int32_t* slots, hipStream_t stream);
+
+/*
  * Decoder-layer kernels around the paged attention, for fp16 / bf16 operands (sums in
  * fp32).  Dense row-major operands, 16-byte aligned.
  *
@@ -487,6 +496,34 @@ int ivakv_linear_rows(const void* x, int64_t ldx, int m, int k, const void* w0, 
                       const void* w1, int n1, void* out1, const void* w2, int n2, void* out2,
                       const void* residual, int norm, const void* norm_weight, float eps,
                       int epilogue, int dtype, hipStream_t stream);
+
+/*
+ * One pre-norm transformer block on a decode step's rows (one token of each of `batch` <= 32
+ * sequences), as five to seven launches enqueued by one call:
+ *   q, k, v = norm1(x) {wq, wk, wv}^T;  o = append + paged attention;  x1 = x + o wo^T;
+ *   out = x1 + (silu(norm2(x1) wup^T) * (norm2(x1) wgate^T)) wdown^T
+ * The parts are ivakv_rms_norm, ivakv_linear_rows and ivakv_decode_append_attn(_fp8) with
+ * their conditions.  Every field is 8 bytes.  `args` points to an
+ * ivakv_block_decode_args.  scratch (16-byte aligned, uninitialised) holds the intermediate
+ * rows: batch * (3 d_model + 2 num_q_heads head_dim + 2 num_kv_heads head_dim + hidden)
+ * elements and 7 * 256 bytes of alignment.
+ * Replaces: TransformerBlock.forward (src/core/transformer.py:81-151) for seq_len 1.
+ */
+typedef struct ivakv_block_decode_args {
+  const void *x, *norm1, *wq, *wk, *wv, *wo, *norm2, *wgate, *wup, *wdown;
+  void* out;
+  void *k_pool, *v_pool, *k_scale, *v_scale;  /* scales: FP8 pools, else null */
+  const int32_t *block_tables, *context_lens;
+  void* scratch;
+  int64_t scratch_bytes;
+  void* workspace;                            /* ivakv_decode_workspace_size */
+  int64_t workspace_bytes;
+  int64_t batch, d_model, num_q_heads, num_kv_heads, head_dim, hidden, block_size, max_blocks,
+      num_pages, window, n_sink, dtype, fp8;
+  double eps1, eps2, scale;
+} ivakv_block_decode_args;
+
+int ivakv_block_decode(const char* args, hipStream_t stream);
 
 #ifdef __cplusplus
 }

@@ -12,7 +12,8 @@ from __future__ import annotations
 
 import ctypes
 import os
-from ctypes import c_float, c_int, c_int64, c_size_t, c_void_p, POINTER
+import struct
+from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p, POINTER
 from pathlib import Path
 from typing import Optional
 
@@ -179,6 +180,11 @@ SIGNATURES = {
         c_int, c_int, c_int,                   # window, n_sink, dtype
         c_void_p,                              # stream
     ]),
+    "ivakv_chunk_slots": (c_int, [
+        c_void_p, c_void_p, c_int, c_int,      # block_tables, context_lens, batch, n
+        c_int, c_int, c_void_p, c_void_p,      # max_blocks, block_size, slots, stream
+    ]),
+    "ivakv_block_decode": (c_int, [c_char_p, c_void_p]),  # packed args, stream
     "ivakv_rms_norm": (c_int, [
         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,  # x, residual, weight, sum, out
         c_int64, c_int, c_float, c_int, c_void_p,  # rows, d, eps, dtype, stream
@@ -208,6 +214,11 @@ SIGNATURES = {
         c_int, c_void_p,                             # dtype, stream
     ]),
 }
+
+
+# ivakv_block_decode_args in include/ivakv.h: 8-byte fields, pointers and integers, then
+# three doubles.
+BLOCK_DECODE = struct.Struct("=34q3d")
 
 
 class IvakvError(RuntimeError):
@@ -257,8 +268,14 @@ def last_error() -> str:
     return msg.decode() if msg else ""
 
 
+_FUNCS: dict = {}
+
+
 def call(name: str, *args) -> None:
     """Calls entry point ``name``; raises IvakvError on a non-zero status."""
-    status = getattr(lib(), name)(*args)
+    fn = _FUNCS.get(name)
+    if fn is None:
+        fn = _FUNCS[name] = getattr(lib(), name)
+    status = fn(*args)
     if status != OK:
         raise IvakvError(name, status, last_error())

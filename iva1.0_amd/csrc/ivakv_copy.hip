@@ -319,10 +319,44 @@ inline unsigned blocks_for(int64_t total, int per_block) {
 
 constexpr int64_t kMaxGrid = 2147483647LL;
 
+// One thread per new token; latency-bound (a few KiB), it takes the place of a host-built
+// list and its synchronous copy.
+__global__ __launch_bounds__(256) void chunk_slots_kernel(const int32_t* bt, const int32_t* ctx,
+                                                          int64_t total, int n, int max_blocks, int bs,
+                                                          int32_t* slots) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const int64_t b = i / n;
+  const int pos = ctx[b] - n + (int)(i - b * n);
+  int slot = -1;
+  if (pos >= 0 && pos / bs < max_blocks) {
+    const int page = bt[b * max_blocks + pos / bs];
+    if (page >= 0) slot = page * bs + pos % bs;
+  }
+  slots[i] = slot;
+}
+
 }  // namespace
 }  // namespace ivakv
 
 using namespace ivakv;
+
+extern "C" int ivakv_chunk_slots(const int32_t* block_tables, const int32_t* context_lens,
+                                 int batch, int n, int max_blocks, int block_size, int32_t* slots,
+                                 hipStream_t stream) {
+  const char* name = "ivakv_chunk_slots";
+  if (batch < 0 || n < 0 || max_blocks < 0 || block_size <= 0)
+    return fail(IVAKV_E_ARG, "%s: bad sizes B=%d n=%d max_blocks=%d block_size=%d", name, batch, n,
+                max_blocks, block_size);
+  const int64_t total = (int64_t)batch * n;
+  if (total > (int64_t)1 << 38) return fail(IVAKV_E_SHAPE, "%s: launch too large", name);
+  if (total == 0) return IVAKV_OK;
+  if (!context_lens || !slots || (max_blocks > 0 && !block_tables))
+    return fail(IVAKV_E_ARG, "%s: null pointer argument", name);
+  chunk_slots_kernel<<<dim3((unsigned)((total + 255) / 256)), 256, 0, stream>>>(
+      block_tables, context_lens, total, n, max_blocks, block_size, slots);
+  return launch_status(name);
+}
 
 extern "C" int ivakv_append(const void* k_new, const void* v_new, int64_t k_tok_stride,
                             int64_t k_head_stride, int64_t v_tok_stride, int64_t v_head_stride,

@@ -9,6 +9,8 @@
 //                      set by its launch and its serial walk along K; here the waves of a
 //                      workgroup split K, so every weight load of a wave is in flight at
 //                      once, and q / k / v, or gate / up, go in one launch.
+#include <string.h>
+
 #include "ivakv_tile.h"
 
 namespace ivakv {
@@ -549,4 +551,71 @@ extern "C" int ivakv_linear_rows(const void* x, int64_t ldx, int m, int k, const
   if (dtype == IVAKV_F16) launch_linear_w<IVAKV_F16>(a, norm != 0, epilogue, stream);
   else launch_linear_w<IVAKV_BF16>(a, norm != 0, epilogue, stream);
   return launch_status(name);
+}
+
+extern "C" int ivakv_block_decode(const char* args, hipStream_t stream) {
+  const char* name = "ivakv_block_decode";
+  if (!args) return fail(IVAKV_E_ARG, "%s: null args", name);
+  ivakv_block_decode_args a;
+  memcpy(&a, args, sizeof(a));
+  const int dtype = (int)a.dtype;
+  int st = check_16bit(name, dtype);
+  if (st != IVAKV_OK) return st;
+  if (a.batch < 0 || a.batch > kLinearMaxRows || a.d_model <= 0 || a.d_model > 1 << 20 ||
+      a.num_q_heads <= 0 || a.num_q_heads > 1 << 16 || a.num_kv_heads <= 0 ||
+      a.num_kv_heads > a.num_q_heads || a.head_dim <= 0 || a.head_dim > 256 || a.hidden <= 0 ||
+      a.hidden > 1 << 24)
+    return fail(IVAKV_E_ARG, "%s: bad sizes", name);
+  if (a.batch == 0) return IVAKV_OK;
+  const int m = (int)a.batch, d = (int)a.d_model;
+  const int nq = (int)(a.num_q_heads * a.head_dim), nkv = (int)(a.num_kv_heads * a.head_dim);
+  const int hidden = (int)a.hidden;
+  // The intermediate rows, each 256-byte aligned in the scratch.
+  char* base = static_cast<char*>(a.scratch);
+  int64_t used = 0;
+  auto take = [&](int n) -> void* {
+    void* p = base + used;
+    used += ((int64_t)m * n * 2 + 255) & ~(int64_t)255;
+    return p;
+  };
+  void *q = take(nq), *k = take(nkv), *v = take(nkv), *o = take(nq), *x1 = take(d), *h = take(hidden),
+       *y = take(d);
+  if (!base || !aligned16(base) || used > a.scratch_bytes)
+    return fail(IVAKV_E_WORKSPACE, "%s: %lld bytes of scratch (16-byte aligned) required, got %lld", name,
+                (long long)used, (long long)(base ? a.scratch_bytes : 0));
+  const int in_norm = m <= kLinearNormRows && d <= kLinearNormMaxK;
+  const void* y1 = in_norm ? a.x : y;
+  if (!in_norm) {
+    st = ivakv_rms_norm(a.x, nullptr, a.norm1, nullptr, y, m, d, (float)a.eps1, dtype, stream);
+    if (st != IVAKV_OK) return st;
+  }
+  st = ivakv_linear_rows(y1, d, m, d, a.wq, nq, q, a.wk, nkv, k, a.wv, nkv, v, nullptr, in_norm,
+                         a.norm1, (float)a.eps1, kPlain, dtype, stream);
+  if (st != IVAKV_OK) return st;
+  const int hq = (int)a.num_q_heads, hkv = (int)a.num_kv_heads, hd = (int)a.head_dim;
+  if (a.fp8)
+    st = ivakv_decode_append_attn_fp8(q, k, v, a.k_pool, a.v_pool, static_cast<float*>(a.k_scale),
+                                      static_cast<float*>(a.v_scale), a.block_tables, a.context_lens, o,
+                                      a.workspace, (size_t)a.workspace_bytes, m, hq, hkv, hd,
+                                      (int)a.block_size, (int)a.max_blocks, (int)a.num_pages,
+                                      (float)a.scale, (int)a.window, (int)a.n_sink, dtype, stream);
+  else
+    st = ivakv_decode_append_attn(q, k, v, a.k_pool, a.v_pool, a.block_tables, a.context_lens, o,
+                                  a.workspace, (size_t)a.workspace_bytes, m, hq, hkv, hd,
+                                  (int)a.block_size, (int)a.max_blocks, (int)a.num_pages,
+                                  (float)a.scale, (int)a.window, (int)a.n_sink, dtype, stream);
+  if (st != IVAKV_OK) return st;
+  st = ivakv_linear_rows(o, nq, m, nq, a.wo, d, x1, nullptr, 0, nullptr, nullptr, 0, nullptr, a.x, 0,
+                         nullptr, 0.f, kResidual, dtype, stream);
+  if (st != IVAKV_OK) return st;
+  const void* y2 = in_norm ? x1 : y;
+  if (!in_norm) {
+    st = ivakv_rms_norm(x1, nullptr, a.norm2, nullptr, y, m, d, (float)a.eps2, dtype, stream);
+    if (st != IVAKV_OK) return st;
+  }
+  st = ivakv_linear_rows(y2, d, m, d, a.wgate, hidden, h, a.wup, hidden, nullptr, nullptr, 0, nullptr,
+                         nullptr, in_norm, a.norm2, (float)a.eps2, kSwiglu, dtype, stream);
+  if (st != IVAKV_OK) return st;
+  return ivakv_linear_rows(h, hidden, m, hidden, a.wdown, d, a.out, nullptr, 0, nullptr, nullptr, 0, nullptr,
+                           x1, 0, nullptr, 0.f, kResidual, dtype, stream);
 }

@@ -53,9 +53,9 @@ import torch.nn.functional as F
 from torch.nn.modules.module import _has_any_global_hook
 
 from .ops import (FP8, LINEAR_MAX_ROWS, LINEAR_NORM_MAX_K, LINEAR_NORM_MAX_ROWS, NORM_MAX_D,
-                  kv_gather, linear_rows, paged_decode_append_attention,
+                  block_decode, kv_gather, linear_rows, paged_decode_append_attention,
                   paged_prefill_attention, rms_norm, rope_, swiglu)
-from .paged_cache import PagedKVCache
+from .paged_cache import OwnPages, PagedKVCache
 
 
 def _cfg(config: Any, name: str, default: Any) -> Any:
@@ -236,15 +236,18 @@ def _plain_dropout(m: nn.Module) -> bool:
     return _plain_module(m, nn.Dropout) and (not m.training or m.p == 0)
 
 
-def _linear_weight(m: nn.Module, x: torch.Tensor) -> Optional[torch.Tensor]:
-    """The weight of a plain bias-free nn.Linear that the linear kernel takes, else None."""
+def _linear_weight(m: nn.Module, x: torch.Tensor, n: Optional[int], k: int
+                   ) -> Optional[torch.Tensor]:
+    """The weight of a plain bias-free nn.Linear of k inputs (and n outputs) on tensors like
+    x that the linear kernel takes, else None."""
     if not _plain_module(m, nn.Linear):
         return None
     p = m._parameters
     w = p.get("weight")
-    if p.get("bias") is not None or not _plain_weight(w, x) or w.shape[0] % 16 or w.shape[1] % 64:
+    if p.get("bias") is not None or not _plain_weight(w, x) or w.dim() != 2:
         return None
-    return w
+    rows, cols = w.shape
+    return w if cols == k and rows % 16 == 0 and k % 64 == 0 and n in (None, rows) else None
 
 
 def _few_rows(x: torch.Tensor) -> bool:
@@ -438,9 +441,21 @@ class PagedAttention(_AttentionBase):
                 return self._split_heads(linear_rows(x, w))
         return super()._project(x)
 
+    def _decodes(self, x, attention_mask, cache) -> bool:
+        """A decode step that block_decode runs whole: one token per sequence onto a plain
+        paged cache of 16-bit pages like x or FP8 pages, causal, without mask or RoPE."""
+        if (attention_mask is not None or type(cache) is not PagedKVCache or x.shape[1] != 1
+                or not self.causal or self.rope or (self.training and self.dropout > 0)):
+            return False
+        pool = cache.pool
+        return ((pool.dtype is x.dtype or pool.fp8) and pool.num_kv_heads == self.n_kv_heads
+                and pool.head_dim == self.head_dim and pool.k_pools[0].device == x.device)
+
     def _qkv_weights(self, x):
-        m = self._modules
-        w = [_linear_weight(m[n], x) for n in ("q_proj", "k_proj", "v_proj")]
+        m, k = self._modules, x.shape[-1]
+        q_dim, kv_dim = self.n_heads * self.head_dim, self.n_kv_heads * self.head_dim
+        w = (_linear_weight(m["q_proj"], x, q_dim, k), _linear_weight(m["k_proj"], x, kv_dim, k),
+             _linear_weight(m["v_proj"], x, kv_dim, k))
         return None if any(t is None for t in w) else w
 
     def _split_heads(self, qkv):
@@ -452,7 +467,7 @@ class PagedAttention(_AttentionBase):
 
     def _output(self, out):
         if _plain_mode() and _plain_input(out) and _few_rows(out) and not _has_any_global_hook():
-            w = _linear_weight(self._modules["o_proj"], out)
+            w = _linear_weight(self._modules["o_proj"], out, None, out.shape[-1])
             if w is not None:
                 return linear_rows(out, (w,))
         return self.o_proj(out)
@@ -468,8 +483,11 @@ class PagedAttention(_AttentionBase):
         b, s, _ = x.shape
         returned = kv_cache
         if kv_cache is None and self.causal:
-            kv_cache = PagedKVCache(b, self.n_kv_heads, self.head_dim, 0, x.device, x.dtype,
-                                    num_layers=1, max_seq_len=s)
+            if x.is_cuda and b * s:
+                kv_cache = OwnPages(b, s, self.n_kv_heads, self.head_dim, x.device, x.dtype)
+            else:
+                kv_cache = PagedKVCache(b, self.n_kv_heads, self.head_dim, 0, x.device, x.dtype,
+                                        num_layers=1, max_seq_len=s)
         q, k, v = project(x)
         n_sink = _sink_count(sink_cfg, self.sink_tokens)
         window = sliding_window if sliding_window and sliding_window > 0 else None
@@ -628,9 +646,13 @@ class FFN(nn.Module):
 
     def _weights(self, x):
         """(gate, up, down) weights when the linear kernel takes all three, else None."""
-        m = self._modules
-        w = [_linear_weight(m[n], x) for n in ("gate_proj", "up_proj", "down_proj")]
-        return None if any(t is None for t in w) else w
+        m, d = self._modules, x.shape[-1]
+        gate = _linear_weight(m["gate_proj"], x, None, d)
+        if gate is None:
+            return None
+        hidden = gate.shape[0]
+        up, down = _linear_weight(m["up_proj"], x, hidden, d), _linear_weight(m["down_proj"], x, None, hidden)
+        return None if up is None or down is None else (gate, up, down)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.activation == "swiglu":
@@ -685,6 +707,23 @@ class TransformerBlock(nn.Module):
                 and _plain_module(n2, RMSNorm) and _plain_dropout(drop)
                 and n1._kernel_takes(x) and n2._kernel_takes(x) and not _has_any_global_hook())
 
+    def _decode_step(self, x, qkv, wo, w, cache, sliding_window, sink_cfg):
+        """The block on one new token per sequence of a paged cache, enqueued by one call; the
+        cache moves as in PagedAttention."""
+        attn, n1, n2 = self._modules["attention"], self._modules["norm1"], self._modules["norm2"]
+        n_sink = _sink_count(sink_cfg, attn.sink_tokens)
+        window = sliding_window if sliding_window and sliding_window > 0 else 0
+        if cache.current_layer == 0:
+            cache.note_window(window or None, n_sink)
+        view = cache._layer_view(x.shape[0], 1)
+        cache._next_layer(view)
+        out = block_decode(x, n1.weight, n1.eps, *qkv, wo, n2.weight, n2.eps, *w, view.k_pool,
+                           view.v_pool, view.block_tables, view.context_lens, attn.n_heads,
+                           attn.scale, window, n_sink if window else 0, **view.scales)
+        if cache.current_layer == 0:
+            cache.release_window()
+        return out, cache
+
     def _forward_fused(self, x, attention_mask, kv_cache, sliding_window, sink_cfg):
         """The block with its norms, residual adds and SwiGLU fused: on a decode step's rows
         into the linear kernel (five launches with the attention), on more rows the residual
@@ -692,9 +731,12 @@ class TransformerBlock(nn.Module):
         m = self._modules
         attn, ffn, n1, n2 = m["attention"], m["ffn"], m["norm1"], m["norm2"]
         if _few_rows(x):
-            qkv, wo = attn._qkv_weights(x), _linear_weight(attn._modules["o_proj"], x)
-            w = ffn._weights(x)
-            if qkv is not None and wo is not None and w is not None:
+            d = x.shape[-1]
+            qkv, w = attn._qkv_weights(x), ffn._weights(x)
+            wo = _linear_weight(attn._modules["o_proj"], x, d, attn.n_heads * attn.head_dim)
+            if qkv is not None and wo is not None and w is not None and w[2].shape[0] == d:
+                if attn._decodes(x, attention_mask, kv_cache):
+                    return self._decode_step(x, qkv, wo, w, kv_cache, sliding_window, sink_cfg)
                 in_norm = (x.numel() <= LINEAR_NORM_MAX_ROWS * x.shape[-1]
                            and x.shape[-1] <= LINEAR_NORM_MAX_K)
 
@@ -768,7 +810,8 @@ class Transformer(nn.Module):
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         w = self.token_embedding.weight if self.lm_head is None else self.lm_head.weight
         if (_plain_mode() and _plain_input(x) and x.numel() <= HEAD_MAX_ROWS * x.shape[-1]
-                and _plain_weight(w, x) and w.shape[0] % 16 == 0 and w.shape[1] % 64 == 0):
+                and _plain_weight(w, x) and w.dim() == 2 and w.shape[1] == x.shape[-1]
+                and w.shape[0] % 16 == 0 and w.shape[1] % 64 == 0):
             return linear_rows(x, (w,))
         return F.linear(x, w)
 

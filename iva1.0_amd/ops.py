@@ -13,7 +13,9 @@ FP8 pools (torch.float8_e4m3fn) carry one fp32 scaling factor per (slot, kv head
 """
 from __future__ import annotations
 
+import ctypes
 import math
+from functools import lru_cache
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -57,7 +59,7 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 def chunk_elems(dtype: torch.dtype) -> int:
     """Elements per 16-byte chunk (the innermost K-page dimension)."""
-    return 16 // torch.empty((), dtype=dtype).element_size()
+    return 16 // dtype.itemsize
 
 
 def pool_shapes(num_pages: int, num_kv_heads: int, head_dim: int, block_size: int,
@@ -80,7 +82,7 @@ def pool_geometry(k_pool: torch.Tensor, v_pool: torch.Tensor) -> Tuple[int, int,
     if x != chunk_elems(k_pool.dtype):
         raise ValueError(f"k_pool innermost dim {x} != 16-byte chunk {chunk_elems(k_pool.dtype)}")
     head_dim = nch * x
-    if tuple(v_pool.shape) != (num_pages, hkv, head_dim, bs):
+    if v_pool.shape != (num_pages, hkv, head_dim, bs):
         raise ValueError(f"v_pool shape {tuple(v_pool.shape)} != {(num_pages, hkv, head_dim, bs)}")
     if k_pool.dtype != v_pool.dtype:
         raise TypeError("k_pool and v_pool dtypes differ")
@@ -92,14 +94,20 @@ def pool_geometry(k_pool: torch.Tensor, v_pool: torch.Tensor) -> Tuple[int, int,
 def _require_gpu(*tensors: torch.Tensor) -> torch.device:
     dev = tensors[0].device
     for t in tensors:
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(f"paged KV ops run on the GPU only; got a tensor on {t.device}")
         if t.device != dev:
             raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
     return dev
 
 
+# The current stream's handle without a Stream object around it, where torch has it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(dev: torch.device) -> int:
+    if _raw_stream is not None and dev.index is not None:
+        return _raw_stream(dev.index)
     return torch.cuda.current_stream(dev).cuda_stream
 
 
@@ -114,6 +122,11 @@ def _i32(t: torch.Tensor, name: str) -> torch.Tensor:
     if t.dtype != torch.int32:
         raise TypeError(f"{name} must be int32, got {t.dtype}")
     return t.contiguous()
+
+
+def _i32_row(t: torch.Tensor, name: str) -> torch.Tensor:
+    t = _i32(t, name)
+    return t if t.dim() == 1 else t.reshape(-1)
 
 
 def _buffer(t: torch.Tensor, dev: torch.device, name: str) -> torch.Tensor:
@@ -145,14 +158,14 @@ def kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_pool: torch.Tensor, v_
                            rope_positions, rope_theta)
     dev = _require_gpu(k_new, v_new, k_pool, v_pool, slot_mapping)
     num_pages, hkv, head_dim, bs = pool_geometry(k_pool, v_pool)
-    if k_new.dim() != 3 or tuple(k_new.shape) != tuple(v_new.shape):
+    if k_new.dim() != 3 or k_new.shape != v_new.shape:
         raise ValueError(f"k_new/v_new must be [n_tok, Hkv, D]; got {tuple(k_new.shape)} and {tuple(v_new.shape)}")
     n_tok = k_new.shape[0]
     if k_new.shape[1:] != (hkv, head_dim):
         raise ValueError(f"new rows are {tuple(k_new.shape[1:])}, pool holds ({hkv}, {head_dim})")
     if k_new.dtype != k_pool.dtype or v_new.dtype != k_pool.dtype:
         raise TypeError(f"new rows dtype {k_new.dtype}/{v_new.dtype} != pool dtype {k_pool.dtype}")
-    slot_mapping = _i32(slot_mapping, "slot_mapping").reshape(-1)
+    slot_mapping = _i32_row(slot_mapping, "slot_mapping")
     if slot_mapping.numel() != n_tok:
         raise ValueError(f"slot_mapping has {slot_mapping.numel()} entries for {n_tok} tokens")
     if n_tok == 0:
@@ -162,7 +175,7 @@ def kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_pool: torch.Tensor, v_
     if v_new.stride(2) != 1:
         v_new = v_new.contiguous()
     if rope_positions is not None:
-        pos = _i32(rope_positions, "rope_positions").reshape(-1)
+        pos = _i32_row(rope_positions, "rope_positions")
         if pos.numel() != n_tok or pos.device != dev:
             raise ValueError(f"rope_positions must be {n_tok} int32 values on {dev}")
         _abi.call("ivakv_append_rope", k_new.data_ptr(), v_new.data_ptr(),
@@ -196,7 +209,7 @@ def kv_gather(k_pool: torch.Tensor, v_pool: torch.Tensor, block_tables: torch.Te
     dev = _require_gpu(k_pool, v_pool, block_tables, context_lens)
     num_pages, hkv, head_dim, bs = pool_geometry(k_pool, v_pool)
     block_tables = _i32(block_tables, "block_tables")
-    context_lens = _i32(context_lens, "context_lens").reshape(-1)
+    context_lens = _i32_row(context_lens, "context_lens")
     if block_tables.dim() != 2 or block_tables.shape[0] != context_lens.numel():
         raise ValueError("block_tables must be [B, max_blocks] with B == len(context_lens)")
     batch, max_blocks = block_tables.shape
@@ -226,10 +239,15 @@ def decode_workspace_bytes(batch: int, num_q_heads: int, num_kv_heads: int, head
                            partition_pages: int = 0) -> int:
     """Workspace bytes :func:`paged_decode_attention` needs (0 when no sequence spans more
     than one partition).  The workspace needs no initialisation."""
-    import ctypes
+    return _decode_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, block_size,
+                                   max_blocks, window, n_sink, partition_pages)
+
+
+@lru_cache(maxsize=1024)
+def _decode_workspace_bytes(*geometry) -> int:
+    """A function of the geometry alone (the plan's sizes)."""
     out = ctypes.c_size_t(0)
-    _abi.call("ivakv_decode_workspace_size", batch, num_q_heads, num_kv_heads, head_dim,
-              block_size, max_blocks, window, n_sink, partition_pages, ctypes.byref(out))
+    _abi.call("ivakv_decode_workspace_size", *geometry, ctypes.byref(out))
     return int(out.value)
 
 
@@ -279,7 +297,6 @@ def prefill_split_workspace_bytes(batch: int, num_q_heads: int, num_kv_heads: in
                                   dtype: torch.dtype) -> int:
     """Workspace bytes of :func:`paged_prefill_attention` with ``split=True`` (its plan
     and 512 fp32 row-block partials).  The workspace needs no initialisation."""
-    import ctypes
     out = ctypes.c_size_t(0)
     _abi.call("ivakv_prefill_split_workspace_size", batch, num_q_heads, num_kv_heads, head_dim,
               max_query_len, dtype_code(dtype), ctypes.byref(out))
@@ -323,7 +340,7 @@ def _decode(entry: str, q, k_pool, v_pool, block_tables, context_lens, scale, wi
         raise ValueError("FP8 pools need k_scale / v_scale")
     batch, hq, _ = q.shape
     block_tables = _i32(block_tables, "block_tables")
-    context_lens = _i32(context_lens, "context_lens").reshape(-1)
+    context_lens = _i32_row(context_lens, "context_lens")
     if block_tables.dim() != 2 or block_tables.shape[0] != batch or context_lens.numel() != batch:
         raise ValueError("block_tables must be [B, max_blocks] and context_lens [B]")
     max_blocks = block_tables.shape[1]
@@ -335,17 +352,19 @@ def _decode(entry: str, q, k_pool, v_pool, block_tables, context_lens, scale, wi
     partition_pages = int(partition_pages) if partition_pages else 0
     if out is None:
         out = torch.empty_like(q)
-    elif tuple(out.shape) != tuple(q.shape) or out.dtype != q.dtype or not out.is_contiguous():
-        raise ValueError("out must be a contiguous tensor shaped and typed like q")
-    _buffer(out, dev, "out")
+    else:
+        if out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
+            raise ValueError("out must be a contiguous tensor shaped and typed like q")
+        _buffer(out, dev, "out")
     nbytes = decode_workspace_bytes(batch, hq, hkv, head_dim, bs, max_blocks, window, n_sink,
                                     partition_pages)
     if workspace is None:
         workspace = _workspace(dev, nbytes)
-    elif workspace.numel() * workspace.element_size() < nbytes:
-        raise ValueError(f"workspace has {workspace.numel() * workspace.element_size()} bytes, "
-                         f"{nbytes} needed")
-    _buffer(workspace, dev, "workspace")
+    else:
+        if workspace.numel() * workspace.element_size() < nbytes:
+            raise ValueError(f"workspace has {workspace.numel() * workspace.element_size()} bytes, "
+                             f"{nbytes} needed")
+        _buffer(workspace, dev, "workspace")
     if scales is not None:
         _abi.call(entry, q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),
                   scales[0].data_ptr(), scales[1].data_ptr(), block_tables.data_ptr(),
@@ -435,7 +454,7 @@ def paged_decode_append_attention(q: torch.Tensor, k_new: torch.Tensor, v_new: t
         raise ValueError(f"q must be [B, Hq, {head_dim}]; got {tuple(q.shape)}")
     batch, hq, _ = q.shape
     for name, t in (("k_new", k_new), ("v_new", v_new)):
-        if tuple(t.shape) != (batch, hkv, head_dim):
+        if t.shape != (batch, hkv, head_dim):
             raise ValueError(f"{name} must be [{batch}, {hkv}, {head_dim}]; got {tuple(t.shape)}")
     fp8 = is_fp8(k_pool)
     for t in (q, k_new, v_new):
@@ -445,7 +464,7 @@ def paged_decode_append_attention(q: torch.Tensor, k_new: torch.Tensor, v_new: t
             raise TypeError(f"dtype {t.dtype} != {q.dtype if fp8 else k_pool.dtype}")
     scales = _scales(k_pool, k_scale, v_scale) if fp8 else None
     block_tables = _i32(block_tables, "block_tables")
-    context_lens = _i32(context_lens, "context_lens").reshape(-1)
+    context_lens = _i32_row(context_lens, "context_lens")
     if block_tables.dim() != 2 or block_tables.shape[0] != batch or context_lens.numel() != batch:
         raise ValueError("block_tables must be [B, max_blocks] and context_lens [B]")
     max_blocks = block_tables.shape[1]
@@ -456,16 +475,18 @@ def paged_decode_append_attention(q: torch.Tensor, k_new: torch.Tensor, v_new: t
     n_sink = int(n_sink) if n_sink else 0
     if out is None:
         out = torch.empty_like(q)
-    elif tuple(out.shape) != tuple(q.shape) or out.dtype != q.dtype or not out.is_contiguous():
-        raise ValueError("out must be a contiguous tensor shaped and typed like q")
-    _buffer(out, dev, "out")
+    else:
+        if out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
+            raise ValueError("out must be a contiguous tensor shaped and typed like q")
+        _buffer(out, dev, "out")
     nbytes = decode_workspace_bytes(batch, hq, hkv, head_dim, bs, max_blocks, window, n_sink)
     if workspace is None:
         workspace = _workspace(dev, nbytes)
-    elif workspace.numel() * workspace.element_size() < nbytes:
-        raise ValueError(f"workspace has {workspace.numel() * workspace.element_size()} bytes, "
-                         f"{nbytes} needed")
-    _buffer(workspace, dev, "workspace")
+    else:
+        if workspace.numel() * workspace.element_size() < nbytes:
+            raise ValueError(f"workspace has {workspace.numel() * workspace.element_size()} bytes, "
+                             f"{nbytes} needed")
+        _buffer(workspace, dev, "workspace")
     if fp8:
         _abi.call("ivakv_decode_append_attn_fp8", q.data_ptr(), k_new.data_ptr(),
                   v_new.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), scales[0].data_ptr(),
@@ -489,7 +510,7 @@ def _append_fp8(k_new, v_new, k_pool, v_pool, slot_mapping, k_scale, v_scale,
     dev = _require_gpu(k_new, v_new, k_pool, v_pool, slot_mapping)
     num_pages, hkv, head_dim, bs = pool_geometry(k_pool, v_pool)
     k_scale, v_scale = _scales(k_pool, k_scale, v_scale)
-    if k_new.dim() != 3 or tuple(k_new.shape) != tuple(v_new.shape):
+    if k_new.dim() != 3 or k_new.shape != v_new.shape:
         raise ValueError(f"k_new/v_new must be [n_tok, Hkv, D]; got {tuple(k_new.shape)} and {tuple(v_new.shape)}")
     n_tok = k_new.shape[0]
     if k_new.shape[1:] != (hkv, head_dim):
@@ -497,7 +518,7 @@ def _append_fp8(k_new, v_new, k_pool, v_pool, slot_mapping, k_scale, v_scale,
     if k_new.dtype != v_new.dtype:
         raise TypeError("k_new and v_new dtypes differ")
     code = dtype_code(k_new.dtype)
-    slot_mapping = _i32(slot_mapping, "slot_mapping").reshape(-1)
+    slot_mapping = _i32_row(slot_mapping, "slot_mapping")
     if slot_mapping.numel() != n_tok:
         raise ValueError(f"slot_mapping has {slot_mapping.numel()} entries for {n_tok} tokens")
     if n_tok == 0:
@@ -507,7 +528,7 @@ def _append_fp8(k_new, v_new, k_pool, v_pool, slot_mapping, k_scale, v_scale,
     if v_new.stride(2) != 1:
         v_new = v_new.contiguous()
     if rope_positions is not None:
-        pos = _i32(rope_positions, "rope_positions").reshape(-1)
+        pos = _i32_row(rope_positions, "rope_positions")
         if pos.numel() != n_tok or pos.device != dev:
             raise ValueError(f"rope_positions must be {n_tok} int32 values on {dev}")
         _abi.call("ivakv_append_rope_fp8", k_new.data_ptr(), v_new.data_ptr(),
@@ -528,7 +549,7 @@ def _gather_fp8(k_pool, v_pool, block_tables, context_lens, out_len, out, k_scal
     num_pages, hkv, head_dim, bs = pool_geometry(k_pool, v_pool)
     k_scale, v_scale = _scales(k_pool, k_scale, v_scale)
     block_tables = _i32(block_tables, "block_tables")
-    context_lens = _i32(context_lens, "context_lens").reshape(-1)
+    context_lens = _i32_row(context_lens, "context_lens")
     if block_tables.dim() != 2 or block_tables.shape[0] != context_lens.numel():
         raise ValueError("block_tables must be [B, max_blocks] with B == len(context_lens)")
     batch, max_blocks = block_tables.shape
@@ -600,8 +621,8 @@ def paged_prefill_attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch
         raise TypeError(f"q dtype {q.dtype} != pool dtype {k_pool.dtype}")
     hq = q.shape[1]
     block_tables = _i32(block_tables, "block_tables")
-    context_lens = _i32(context_lens, "context_lens").reshape(-1)
-    query_start = _i32(query_start, "query_start").reshape(-1)
+    context_lens = _i32_row(context_lens, "context_lens")
+    query_start = _i32_row(query_start, "query_start")
     batch = context_lens.numel()
     if block_tables.dim() != 2 or block_tables.shape[0] != batch:
         raise ValueError("block_tables must be [B, max_blocks] with B == len(context_lens)")
@@ -623,9 +644,10 @@ def paged_prefill_attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch
     n_sink = int(n_sink) if n_sink else 0
     if out is None:
         out = torch.empty_like(q)
-    elif tuple(out.shape) != tuple(q.shape) or out.dtype != q.dtype or not out.is_contiguous():
-        raise ValueError("out must be a contiguous tensor shaped and typed like q")
-    _buffer(out, dev, "out")
+    else:
+        if out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
+            raise ValueError("out must be a contiguous tensor shaped and typed like q")
+        _buffer(out, dev, "out")
     max_blocks = block_tables.shape[1]
     if split is None:
         split = prefill_split_default(batch, hq, hkv, q.shape[0], int(max_query_len), max_blocks,
@@ -684,6 +706,23 @@ def rope_(x: torch.Tensor, positions: torch.Tensor, theta: float = 10000.0) -> t
     _abi.call("ivakv_rope", x.data_ptr(), x.stride(0), x.stride(1), pos.data_ptr(), x.shape[0],
               x.shape[1], x.shape[2], float(theta), dtype_code(x.dtype), _stream(dev))
     return x
+
+
+def chunk_slots(block_tables: torch.Tensor, context_lens: torch.Tensor, n: int,
+                block_size: int = 16) -> torch.Tensor:
+    """int32 ``[B * n]`` slots of the last ``n`` positions of each sequence, token-major: the
+    ``slot_mapping`` of :func:`kv_append` for ``n`` new tokens per sequence that the tables
+    and lengths already include.  -1 where a position has no page."""
+    dev = _require_gpu(block_tables, context_lens)
+    block_tables = _i32(block_tables, "block_tables")
+    context_lens = _i32_row(context_lens, "context_lens")
+    batch = context_lens.numel()
+    if block_tables.dim() != 2 or block_tables.shape[0] != batch:
+        raise ValueError("block_tables must be [B, max_blocks] with B == len(context_lens)")
+    out = torch.empty(batch * n, dtype=torch.int32, device=dev)
+    _abi.call("ivakv_chunk_slots", block_tables.data_ptr(), context_lens.data_ptr(), batch, n,
+              block_tables.shape[1], block_size, out.data_ptr(), _stream(dev))
+    return out
 
 
 # Decoder-layer kernels (ivakv_layer.hip).  The callers in model.py check that the operands
@@ -745,6 +784,36 @@ def linear_rows(x: torch.Tensor, weights, norm=None, residual: Optional[torch.Te
               2 if swiglu_pair else 1 if residual is not None else 0, dtype_code(x.dtype),
               _stream(x.device))
     return outs if len(outs) > 1 else outs[0]
+
+
+def block_decode(x: torch.Tensor, norm1, eps1: float, wq, wk, wv, wo, norm2, eps2: float, wgate, wup,
+                 wdown, k_pool, v_pool, block_tables, context_lens, num_q_heads: int, scale: float,
+                 window: int, n_sink: int, k_scale=None, v_scale=None) -> torch.Tensor:
+    """One pre-norm transformer block on a decode step's rows ``x [B, 1, d_model]`` (ivakv_block_decode:
+    every launch of the block from one call).  The new K/V rows go to position
+    ``context_lens[b] - 1``.  Operands as the callers of :func:`linear_rows` check them."""
+    dev = x.device
+    m, d = x.numel() // x.shape[-1], x.shape[-1]
+    num_pages, hkv, head_dim, bs = pool_geometry(k_pool, v_pool)
+    fp8 = is_fp8(k_pool)
+    if fp8:
+        _scales(k_pool, k_scale, v_scale)
+    hidden, max_blocks = wup.shape[0], block_tables.shape[1]
+    out = torch.empty_like(x)
+    ws = _workspace(dev, decode_workspace_bytes(m, num_q_heads, hkv, head_dim, bs, max_blocks, window,
+                                                n_sink))
+    nbytes = 2 * m * (3 * d + 2 * (num_q_heads + hkv) * head_dim + hidden) + 7 * 256
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    args = _abi.BLOCK_DECODE.pack(
+        x.data_ptr(), 0 if norm1 is None else norm1.data_ptr(), wq.data_ptr(), wk.data_ptr(),
+        wv.data_ptr(), wo.data_ptr(), 0 if norm2 is None else norm2.data_ptr(), wgate.data_ptr(),
+        wup.data_ptr(), wdown.data_ptr(), out.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),
+        k_scale.data_ptr() if fp8 else 0, v_scale.data_ptr() if fp8 else 0, block_tables.data_ptr(),
+        context_lens.data_ptr(), scratch.data_ptr(), nbytes, ws.data_ptr(), ws.numel(), m, d, num_q_heads,
+        hkv, head_dim, hidden, bs, max_blocks, num_pages, window, n_sink, dtype_code(x.dtype), int(fp8),
+        eps1, eps2, scale)
+    _abi.call("ivakv_block_decode", args, _stream(dev))
+    return out
 
 
 def copy_pages(k_pool: torch.Tensor, v_pool: torch.Tensor, src_pages: torch.Tensor,

@@ -31,7 +31,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 import numpy as np
 import torch
 
-from .ops import FP8, copy_pages, kv_append, kv_gather, pool_shapes, scale_shape
+from .ops import FP8, chunk_slots, copy_pages, kv_append, kv_gather, pool_shapes, scale_shape
 
 
 class OutOfPagesError(RuntimeError):
@@ -229,6 +229,16 @@ class PagedKVPool:
         self.context_lens[self._rows[seq_id]] = s.length
         return self.slots(seq_id, np.arange(start, s.length))
 
+    def extend(self, seq_ids: Sequence, n_tokens: int) -> None:
+        """:meth:`allocate` of ``n_tokens`` for each sequence in turn, without the slot ids."""
+        n = int(n_tokens)
+        for seq_id in seq_ids:
+            s = self._seq(seq_id)
+            if n < 0 or s.length + n > len(s.pages) * self.block_size:
+                self.reserve(seq_id, n)
+            s.length += n
+            self.context_lens[self._rows[seq_id]] = s.length
+
     def free(self, seq_id) -> None:
         """Returns the sequence's pages to the free list (shared pages stay until their
         last owner frees them) and releases its block-table row."""
@@ -366,18 +376,37 @@ class PagedKVPool:
             self._sync_row(k)
 
 
+class _Slots:
+    """The slot mapping of a forward's new tokens, computed on the device when first needed
+    (the fused decode step finds its slots itself)."""
+
+    def __init__(self, block_tables, context_lens, n: int, block_size: int):
+        self._args = (block_tables, context_lens, n, block_size)
+        self._slots: Optional[torch.Tensor] = None
+
+    def get(self) -> torch.Tensor:
+        if self._slots is None:
+            self._slots = chunk_slots(*self._args)
+        return self._slots
+
+
 @dataclass
 class LayerView:
     """What one attention layer of one forward gets from a PagedKVCache."""
     layer: int
     k_pool: torch.Tensor
     v_pool: torch.Tensor
-    slot_mapping: torch.Tensor   # int32 [B * T], token-major (b, t)
+    slots: "torch.Tensor | _Slots"
     block_tables: torch.Tensor   # int32 [B, max_blocks]
     context_lens: torch.Tensor   # int32 [B], lengths after this forward's append
     start: int                   # position of the first new token
     new_tokens: int              # T
     scales: Dict[str, torch.Tensor] = field(default_factory=dict)  # FP8: k_scale / v_scale
+
+    @property
+    def slot_mapping(self) -> torch.Tensor:
+        """int32 [B * T], token-major (b, t)."""
+        return self.slots.get() if isinstance(self.slots, _Slots) else self.slots
 
 
 class PagedKVCache:
@@ -581,12 +610,24 @@ class PagedKVCache:
     def _tables(self) -> Tuple[torch.Tensor, torch.Tensor]:
         """Device block table (copied again only when the pool's tables changed since the
         last copy) and context lengths of this cache's sequences."""
-        bt, ctx = self.pool.tables(self.seq_ids)
-        gen = self.pool.generation
-        if self._bt_dev is None or self._bt_gen != gen or self._bt_dev.shape != bt.shape:
-            self._bt_dev = torch.from_numpy(bt).to(self.device)
-            self._bt_gen = gen
-        return self._bt_dev, torch.from_numpy(ctx).to(self.device)
+        pool = self.pool
+        if self._bt_dev is None or self._bt_gen != pool.generation:
+            bt, _ = pool.tables(self.seq_ids)
+            self._bt_dev = self._to_device(bt)
+            self._bt_gen = pool.generation
+        ctx = pool.context_lens[[pool.row(s) for s in self.seq_ids]]
+        if len(ctx) and (ctx == ctx[0]).all():  # the batch in step, the usual case: no copy
+            return self._bt_dev, torch.full((len(ctx),), int(ctx[0]), dtype=torch.int32,
+                                            device=self.device)
+        return self._bt_dev, self._to_device(ctx)
+
+    def _to_device(self, a: np.ndarray) -> torch.Tensor:
+        """A host array on the device, copied through pinned memory where there is a GPU, so
+        that the host does not wait for the stream's earlier work."""
+        t = torch.from_numpy(np.ascontiguousarray(a))
+        if self.device.type != "cuda":
+            return t.to(self.device)
+        return t.pin_memory().to(self.device, non_blocking=True)
 
     # ------------------------------------------------------ static decode
     @property
@@ -671,7 +712,20 @@ class PagedKVCache:
         ``seq_len`` by T and rewinds the cursor.  ``append=False`` allocates and
         advances the same way but leaves writing the rows to the caller (the fused
         decode op writes them itself)."""
-        b, t = k_rows.shape[0], k_rows.shape[1]
+        view = self._layer_view(k_rows.shape[0], k_rows.shape[1])
+        if append:
+            b, t = k_rows.shape[0], k_rows.shape[1]
+            rope = {} if rope_positions is None else {"rope_positions": rope_positions,
+                                                      "rope_theta": rope_theta}
+            kv_append(k_rows.reshape(b * t, self.n_heads, self.head_dim),
+                      v_rows.reshape(b * t, self.n_heads, self.head_dim),
+                      view.k_pool, view.v_pool, view.slot_mapping, **view.scales, **rope)
+        self._next_layer(view)
+        return view
+
+    def _layer_view(self, b: int, t: int) -> LayerView:
+        """The view of the layer at the cursor for ``t`` new tokens of ``b`` sequences, which
+        the first layer allocates."""
         if b != self.batch_size:
             raise ValueError(f"batch {b} != cache batch {self.batch_size}")
         if self._cursor == 0 and self._static is not None:
@@ -680,31 +734,24 @@ class PagedKVCache:
             self._view = self._static_step()
         elif self._cursor == 0:
             start = self.seq_len
-            slots = np.concatenate([self.pool.allocate(s, t) for s in self.seq_ids])
-            slot_dev = torch.from_numpy(slots).to(self.device, non_blocking=True)
+            self.pool.extend(self.seq_ids, t)
             bt, ctx = self._tables()
-            self._view = (slot_dev, bt, ctx, start, t)
+            self._view = (_Slots(bt, ctx, t, self.block_size), bt, ctx, start, t)
         elif self._view is None or self._view[4] != t:
             raise RuntimeError("layer cursor out of step: every layer of a forward must append "
                                "the same tokens")
-        slot_dev, bt, ctx, start, t = self._view
+        slots, bt, ctx, start, t = self._view
         layer = self._cursor
-        if append:
-            rope = {} if rope_positions is None else {"rope_positions": rope_positions,
-                                                      "rope_theta": rope_theta}
-            kv_append(k_rows.reshape(b * t, self.n_heads, self.head_dim),
-                      v_rows.reshape(b * t, self.n_heads, self.head_dim),
-                      self.pool.k_pools[layer], self.pool.v_pools[layer], slot_dev,
-                      **self.pool.scales(layer), **rope)
-        view = LayerView(layer, self.pool.k_pools[layer], self.pool.v_pools[layer], slot_dev, bt,
-                         ctx, start, t, self.pool.scales(layer))
+        return LayerView(layer, self.pool.k_pools[layer], self.pool.v_pools[layer], slots, bt, ctx,
+                         start, t, self.pool.scales(layer))
+
+    def _next_layer(self, view: LayerView) -> None:
         self._cursor += 1
         if self._cursor == self.num_layers:
             self._cursor = 0
             if self._static is None:
-                self.seq_len = start + t
+                self.seq_len = view.start + view.new_tokens
             self._view = None
-        return view
 
     def reset_cursor(self) -> None:
         """Rewinds the layer cursor after a forward that did not reach the last layer
@@ -727,6 +774,44 @@ class PagedKVCache:
                   torch.from_numpy(slots).to(self.device), **self.pool.scales(layer_only))
         if commit:
             self.seq_len = t
+
+
+class OwnPages:
+    """The pages of one attention layer's own tokens, for a forward without a cache: ``batch``
+    sequences of ``tokens`` new tokens, sequence b on pages b * n .. (b + 1) * n - 1.  What
+    a one-layer PagedKVCache of those tokens would hand out, with tables and slots made on
+    the device (no host bookkeeping or copy) and pools left uninitialised past the tokens,
+    which no kernel reads unmasked."""
+
+    current_layer = 0
+
+    def __init__(self, batch: int, tokens: int, n_heads: int, head_dim: int, device, dtype):
+        self.batch, self.tokens, self.n_heads, self.head_dim = batch, tokens, n_heads, head_dim
+        per = -(-tokens // 16)
+        ks, vs = pool_shapes(batch * per, n_heads, head_dim, 16, dtype)
+        tables = torch.arange(batch * per, dtype=torch.int32, device=device).view(batch, per)
+        lens = torch.full((batch,), tokens, dtype=torch.int32, device=device)
+        self.fp8 = False
+        self.pool = self
+        self._view = LayerView(0, torch.empty(ks, dtype=dtype, device=device),
+                               torch.empty(vs, dtype=dtype, device=device),
+                               _Slots(tables, lens, tokens, 16), tables, lens, 0, tokens)
+
+    def note_window(self, window, n_sink: int = 0) -> None:
+        pass
+
+    def token_positions(self, t: int) -> torch.Tensor:
+        return torch.arange(t, dtype=torch.int32, device=self._view.context_lens.device).repeat(self.batch)
+
+    def layer_step(self, k_rows, v_rows, append: bool = True, rope_positions=None,
+                   rope_theta: float = 10000.0) -> LayerView:
+        if append:
+            rope = {} if rope_positions is None else {"rope_positions": rope_positions,
+                                                      "rope_theta": rope_theta}
+            shape = (self.batch * self.tokens, self.n_heads, self.head_dim)
+            kv_append(k_rows.reshape(shape), v_rows.reshape(shape), self._view.k_pool,
+                      self._view.v_pool, self._view.slot_mapping, **rope)
+        return self._view
 
 
 def create_kv_cache(batch_size: int, n_heads: int, head_dim: int, seq_len: int,

@@ -276,3 +276,32 @@ def test_layer_kernel_argument_checks(iva):
                 dict(epilogue=1, n=(16, 0, 0)), dict(w=None)):
         assert linear(**bad) == a.E_ARG, bad
     assert linear(m=0) == a.OK
+
+
+def test_block_decode_and_chunk_slots_argument_checks(iva):
+    a = iva._abi
+    assert call(iva, "ivakv_chunk_slots", FAKE, FAKE, -1, 1, 4, 16, FAKE, None) == a.E_ARG
+    assert call(iva, "ivakv_chunk_slots", None, FAKE, 2, 1, 4, 16, FAKE, None) == a.E_ARG
+    assert call(iva, "ivakv_chunk_slots", None, None, 0, 1, 4, 16, None, None) == a.OK
+    names = (["x", "norm1", "wq", "wk", "wv", "wo", "norm2", "wgate", "wup", "wdown", "out", "k_pool", "v_pool",
+              "k_scale", "v_scale", "block_tables", "context_lens", "scratch", "scratch_bytes", "workspace",
+              "workspace_bytes", "batch", "d_model", "num_q_heads", "num_kv_heads", "head_dim", "hidden",
+              "block_size", "max_blocks", "num_pages", "window", "n_sink", "dtype", "fp8"])
+    text = HEADER.read_text().split("typedef struct ivakv_block_decode_args {")[1].split("}")[0]
+    fields = re.findall(r"\*?(\w+)(?=[,;])", re.sub(r"/\*.*?\*/", "", text, flags=re.S))
+    assert fields == names + ["eps1", "eps2", "scale"]
+    good = dict.fromkeys(names, FAKE)
+    good.update(k_scale=0, v_scale=0, scratch_bytes=1 << 20, workspace_bytes=1 << 30, batch=4, d_model=64,
+                num_q_heads=1, num_kv_heads=1, head_dim=64, hidden=256, block_size=16, max_blocks=4, num_pages=8,
+                window=0, n_sink=0, dtype=a.BF16, fp8=0)
+
+    def block(**over):
+        v = {**good, **over}
+        return call(iva, "ivakv_block_decode", a.BLOCK_DECODE.pack(*(v[n] for n in names), 1e-6, 1e-6, 0.1), None)
+
+    assert call(iva, "ivakv_block_decode", None, None) == a.E_ARG
+    assert block(dtype=a.F32) == a.E_DTYPE
+    assert block(batch=33) == block(hidden=0) == block(num_kv_heads=2) == a.E_ARG
+    assert block(scratch_bytes=64) == block(scratch=0) == a.E_WORKSPACE
+    assert block(d_model=96) == a.E_SHAPE and block(wq=0) == a.E_ARG
+    assert block(batch=0) == a.OK

@@ -124,3 +124,57 @@ def test_fused_block_matches_modules(iva, dev, d_model, heads, kv, batch, tokens
     # both round every intermediate once or twice to bf16, six in a row
     err = (fused.double() - alone.double()).norm() / alone.double().norm()
     assert err <= 6 * U[torch.bfloat16], err
+
+
+@pytest.mark.parametrize("kw", [{}, dict(kv_cache_dtype="fp8"), dict(sliding_window=48, sink_tokens=4),
+                                dict(n_kv_heads=1)])
+@pytest.mark.parametrize("batch", [1, 16, 19])
+def test_decode_step_in_one_call_matches_modules(iva, dev, batch, kw):
+    """Decode steps whose blocks are one call each, and the same steps module by module (a
+    hook on a submodule of every block), from the same cached prompt across a page boundary."""
+    M = iva.model
+    cfg = M.TransformerConfig(d_model=512, n_heads=8, **{"n_kv_heads": 2, **kw}, n_layers=3, vocab_size=64,
+                              seq_len=256, dropout=0.1, attn_impl="hip_paged")
+    torch.manual_seed(7)
+    model = M.Transformer(cfg).to(dev, torch.bfloat16).eval()
+    ids = torch.randint(0, 64, (batch, 61 + 5), device=dev, generator=torch.Generator(dev).manual_seed(1))
+
+    def steps():
+        cache = model.new_kv_cache(batch, 66)
+        out = [model(ids[:, :61], kv_cache=cache)["logits"][:, -1]]
+        for t in range(61, 66):
+            out.append(model(ids[:, t:t + 1], kv_cache=cache)["logits"][:, -1])
+        kv = [cache.layer_kv(i) for i in range(3)]
+        n = cache.seq_len
+        cache.free()
+        return torch.stack(out), kv, n
+
+    with torch.no_grad():
+        fused, kv, n = steps()
+        calls = []
+        hooks = [b.ffn.up_proj.register_forward_hook(lambda m, i, o: calls.append(1)) for b in model.blocks]
+        alone, kv2, n2 = steps()
+        for h in hooks:
+            h.remove()
+    assert len(calls) == 3 * 6 and n == n2 == 66
+    # three blocks of about six bf16 roundings in a row (FP8 codes flip at their 2^-4 steps)
+    tol = 18 * U[torch.bfloat16] * (4 if cfg.kv_cache_dtype else 1)
+    for a, b in [(fused, alone)] + [(x, y) for p, q in zip(kv, kv2) for x, y in zip(p, q)]:
+        assert (a.double() - b.double()).norm() <= tol * b.double().norm()
+
+
+@pytest.mark.parametrize("lengths,n", [([16, 16], 16), ([40, 40, 40], 1), ([33, 5, 100], 7), ([3], 5)])
+def test_chunk_slots_match_the_pool(iva, dev, lengths, n):
+    """Slots found on the device equal the allocator's; positions without a page give -1."""
+    pool = iva.PagedKVPool(64, 1, 64, num_layers=1, dtype=torch.float16, device=dev, max_seqs=8)
+    want = []
+    for i, length in enumerate(lengths):
+        pool.add_sequence(i)
+        pool.allocate(i, length)
+        first = max(length - n, 0)
+        want += [-1] * (n - (length - first)) + pool.slots(i, range(first, length)).tolist()
+    bt, ctx = pool.device_tables(range(len(lengths)))
+    assert iva.ops.chunk_slots(bt, ctx, n).tolist() == want
+    assert iva.ops.chunk_slots(bt[:, :1].contiguous(), ctx, 1).tolist() == [
+        pool.slots(i, [length - 1])[0] if length <= 16 else -1 for i, length in enumerate(lengths)]
+    assert iva.ops.chunk_slots(bt, ctx, 0).numel() == 0
