@@ -45,12 +45,17 @@ constexpr int kPageBufs = 2;  // register page buffers per wave (ring)
 constexpr int partial_wgs_per_cu(int D) { return D == 256 ? 1 : 2; }
 // Stream walk workgroup: kStreamWaves independent waves, one per SIMD; how many
 // workgroups share a CU is a property of the tile operations (Ops::kWGsPerCU).
-// Then the wave budget the workspace is sized for, the fewest tiles worth giving
-// a wave, and the largest batch whose page prefix fits the workgroup's LDS.
+// Then the wave budget the workspace is sized for and the largest batch whose page prefix
+// fits the workgroup's LDS.
 constexpr int kStreamWaves = 4;
 constexpr int kStreamThreads = 64 * kStreamWaves;
 constexpr int kMaxStreamWaves = 4096;
-constexpr int kMinTilesPerWave = 4;
+// Fewest tiles worth giving a wave: two (a ring's worth) while that makes at most kFewWaves
+// waves (8 units of 64 pages 12.9 -> 11.2 us, 64 units of <= 48 pages 14.7 -> 13.6 us against
+// four each), four from there (64 units of <= 96 pages 15.6 us, 16.4 at two or three).
+constexpr int kMinTilesPerWave = 2;
+constexpr int kTilesPerWave = 4;
+constexpr int kFewWaves = 800;
 constexpr int kMaxStreamBatch = 8192;
 // Stream walk workgroups per CU from the bytes one ring slot holds (K + V of one
 // tile).  One 4-wave workgroup per CU keeps 2 x 8 KiB slots per wave in flight at
@@ -400,10 +405,12 @@ struct TileOps8 {
 
 // Wave w of partition `part` owns effective pages part*part_pages + w + 4*i,
 // i = 0 .. n_mine-1, and streams them through a ring of kPageBufs register
-// page buffers.  Loads are never skipped: past the wave's last page the index
-// is clamped to that page (an L2 hit) and the duplicate is fully masked, so the
-// loop body has no branches and the compiler's vmcnt waits only cover the
-// buffer about to be consumed.
+// page buffers.  Loads are never skipped: past the wave's last page they read page 0 (as for
+// an invalid page id; every wave's padding reads that tile, an L2 hit, where its own last
+// tile, loaded for streaming, would miss) and the slot is fully masked, so the loop body has
+// no branches and the compiler's vmcnt waits only cover the buffer about to be consumed.  The
+// last round of the ring loads nothing: with it (two more tiles per wave and unit) 256 units
+// of 32 pages took 18.3 us of the 15.7 they take without.
 //
 // Built for two workgroups per CU (one at head_dim 256): with a higher
 // occupancy target the scheduler sinks each load next to its use and the ring
@@ -478,20 +485,26 @@ __global__ __launch_bounds__(kThreads, partial_wgs_per_cu(D)) void decode_partia
   if (n_mine > 0) {
     typename Ops::TileReg tb[kPageBufs];
     int64_t pb[kPageBufs];
-#pragma unroll
-    for (int s = 0; s < kPageBufs; ++s) {
-      pb[s] = phys_page(a, bt, b, logical_page(w, eff_page(s)));
+    auto issue = [&](int s, int i) IVAKV_INLINE {
+      const int64_t p = phys_page(a, bt, b, logical_page(w, eff_page(i)));
+      pb[s] = i < n_mine ? p : -1;
       Ops::load_tile(a, pb[s], h, ln, lq, tb[s]);
-    }
-    for (int i = 0; i < n_mine; i += kPageBufs) {
+    };
+    auto score = [&](int s, int i) IVAKV_INLINE {
+      Ops::score(st, tb[s], qr, w, logical_page(w, eff_page(i)), pb[s] >= 0, a, lq);
+    };
+#pragma unroll
+    for (int s = 0; s < kPageBufs; ++s) issue(s, s);
+    int i = 0;
+    for (; i + kPageBufs < n_mine; i += kPageBufs) {
 #pragma unroll
       for (int s = 0; s < kPageBufs; ++s) {
-        Ops::score(st, tb[s], qr, w, logical_page(w, eff_page(i + s)),
-                   i + s < n_mine && pb[s] >= 0, a, lq);
-        pb[s] = phys_page(a, bt, b, logical_page(w, eff_page(i + s + kPageBufs)));
-        Ops::load_tile(a, pb[s], h, ln, lq, tb[s]);
+        score(s, i + s);
+        issue(s, i + s + kPageBufs);
       }
     }
+#pragma unroll
+    for (int s = 0; s < kPageBufs; ++s) score(s, i + s);
   }
 
   const float l_tot = st.total();
@@ -776,9 +789,13 @@ __device__ inline int64_t div_nn(int64_t n, int64_t d) {
   return n / d;
 }
 
-// Waves that share T tiles: every wave gets at least kMinTilesPerWave.
+// Waves that share T tiles: kMinTilesPerWave each, which is one round trip of the ring, up to
+// kFewWaves waves; beyond that many the partials' merge costs more than the shorter walks
+// save, until every wave has kTilesPerWave.
 __device__ inline int64_t stream_waves(int64_t T, int n_waves) {
-  const int64_t want = (T + kMinTilesPerWave - 1) / kMinTilesPerWave;
+  const int64_t few = (T + kMinTilesPerWave - 1) / kMinTilesPerWave;
+  const int64_t many = (T + kTilesPerWave - 1) / kTilesPerWave;
+  const int64_t want = few <= kFewWaves ? few : many > kFewWaves ? many : kFewWaves;
   return want < n_waves ? (want > 0 ? want : 1) : n_waves;
 }
 
@@ -1315,24 +1332,62 @@ int stream_workgroups(int per_cu) {
   return wgs < kMaxStreamWaves / kStreamWaves ? wgs : kMaxStreamWaves / kStreamWaves;
 }
 
-// Fused calls on short tables whose batch has one to four (sequence, kv head) units
-// per CU take one partition per sequence: a workgroup per unit walks it, merges its
-// waves in LDS, folds the new token and writes out, with no merge kernel (C3's
-// decode shape: 9.9 against 14.9 us for walk + merge; 512 units of 32 / 63 pages
-// 28.4 / 49.1 against 32.4 / 52.9 us).  From four units per CU the stream walk's even
-// shares win (1024 units: 54.6 / 94.9 against 57.2 / 98.7 us; 2048: 102.7 / 182.8
-// against 115.8 / 204.0 us).  Returns the partition size for that, or 0 for the
-// stream walk.
+// Calls on short tables take one partition per sequence: a workgroup per (sequence, kv head)
+// unit walks it, merges its waves in LDS, folds the new token and writes out, with no merge
+// kernel.  Returns the partition size for that, or 0 for the stream walk.
+//   From one unit per CU: tables up to 64 pages.  us, single launch against walk + merge, 8 kv
+//   heads, D 128, all at the table's width / lengths spread from 1 to it: 256 units of 32
+//   pages 15.7 : 19.8 / 13.1 : 18.6, of 64 26.0 : 29.8 / 19.7 : 23.6; 512 of 64 45.3 : 50.7 / 31.4 :
+//   38.3; 1024 of 32 49.3 : 52.7 / 33.0 : 41.7; 2048 of 16 57.3 : 59.3 / 38.3 : 47.6; FP8 1024 of 64
+//   52.3 : 59.0 / 40.7 : 46.0.  Wider tables tell too little of the lengths: at 96 pages the two
+//   meet (256 units spread to 96: 25.9 : 27.9), past them one long unit's walk by one workgroup
+//   would set the time.
+//   Fewer units than CUs: one CU reads about 50 GB/s, so the walk by one workgroup stays ahead
+//   of the stream walk's fixed 11 us only up to kSingleUnitBytes of K and V (32 tiles of 8 KiB:
+//   10.2 - 11.0 against 11.0 - 13.3 us; 48: 12.8 - 13.6 against 11.2 - 13.6), and smaller tiles do
+//   not come faster (FP8, 48 tiles of 4 KiB: 11.9 against 11.5).
 constexpr int kSinglePartitionMaxPages = 64;
-int single_partition_pages(int batch, int num_kv_heads, int max_blocks, int window, int n_sink) {
-  const int max_eff = max_effective_pages(max_blocks, window, n_sink, kBS);
-  if (max_eff <= 0 || max_eff > kSinglePartitionMaxPages || batch > 65535) return 0;
+constexpr int kSingleFewMaxPages = 32;
+constexpr int64_t kSingleUnitBytes = 256 * 1024;
+int device_cus() {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return 0;
-  const int64_t units = (int64_t)batch * num_kv_heads;
-  return units >= cus && units < 4 * (int64_t)cus ? max_eff : 0;
+  return cus;
+}
+int single_partition_pages(int batch, int num_kv_heads, int head_dim, int esize, int max_blocks,
+                           int window, int n_sink) {
+  const int max_eff = max_effective_pages(max_blocks, window, n_sink, kBS);
+  const int cus = device_cus();
+  if (max_eff <= 0 || batch > kMaxStreamBatch || cus <= 0) return 0;
+  int64_t limit = kSinglePartitionMaxPages;
+  if ((int64_t)batch * num_kv_heads < cus) {
+    limit = kSingleUnitBytes / (2 * (int64_t)kBS * head_dim * esize);
+    if (limit > kSingleFewMaxPages) limit = kSingleFewMaxPages;
+  }
+  return max_eff <= limit ? max_eff : 0;
+}
+
+// Plan of a full or fused decode.  A workspace is asked for by the geometry, whichever walk
+// runs: the stream walk's, except for one to four units per CU on tables of at most
+// kSinglePartitionMaxPages.
+int make_decode_plan(const char* name, Stage stage, int batch, int num_q_heads, int num_kv_heads,
+                     int head_dim, int block_size, int max_blocks, int window, int n_sink, int esize,
+                     Plan* plan) {
+  int st = make_plan(name, stage, batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks,
+                     window, n_sink, 0, plan);
+  const int pp = block_size == kBS && n_sink >= 0 && num_kv_heads > 0 && head_dim > 0
+                     ? single_partition_pages(batch, num_kv_heads, head_dim, esize, max_blocks, window, n_sink)
+                     : 0;
+  if (pp <= 0) return st;
+  const size_t stream_bytes = plan->ws_bytes;
+  st = make_plan(name, stage, batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks, window,
+                 n_sink, pp, plan);
+  if (st != IVAKV_OK) return st;
+  const int64_t units = (int64_t)batch * num_kv_heads, cus = device_cus();
+  if (units < cus || units >= 4 * cus) plan->ws_bytes = stream_bytes;
+  return IVAKV_OK;
 }
 
 int decode_entry(Stage stage, const char* name, const void* q, const void* k_pool,
@@ -1352,14 +1407,12 @@ int decode_entry(Stage stage, const char* name, const void* q, const void* k_poo
     if (batch > 0 && (!k_scale || !v_scale || !aligned16(k_scale) || !aligned16(v_scale)))
       return fail(IVAKV_E_ARG, "%s: k_scale / v_scale must be 16-byte aligned device pointers", name);
   }
-  // The single launch for a full decode too (attention alone, the same kernel with no new
-  // token): 256 units of 32 pages 18.3 -> 14.4 us, C3's layer shape 14.1 -> 9.8 us.
-  if ((stage == kFused || stage == kFull) && partition_pages <= 0 && block_size == kBS &&
-      n_sink >= 0)
-    partition_pages = single_partition_pages(batch, num_kv_heads, max_blocks, window, n_sink);
   Plan plan;
-  int st = make_plan(name, stage, batch, num_q_heads, num_kv_heads, head_dim, block_size,
-                     max_blocks, window, n_sink, partition_pages, &plan);
+  int st = (stage == kFused || stage == kFull) && partition_pages <= 0
+               ? make_decode_plan(name, stage, batch, num_q_heads, num_kv_heads, head_dim, block_size,
+                                  max_blocks, window, n_sink, fp8 ? 1 : dtype_size(dtype), &plan)
+               : make_plan(name, stage, batch, num_q_heads, num_kv_heads, head_dim, block_size,
+                           max_blocks, window, n_sink, partition_pages, &plan);
   if (st != IVAKV_OK) return st;
   if (batch == 0) return IVAKV_OK;
   // An invalid page id is read as page 0 (then masked), so the pool needs a page.
@@ -1385,8 +1438,8 @@ int decode_entry(Stage stage, const char* name, const void* q, const void* k_poo
   a.ctx = context_lens;
   a.out = out;
   float* ws = static_cast<float*>(workspace);
-  a.ws_acc = plan.ws_bytes ? ws : nullptr;
-  a.ws_ml = plan.ws_bytes ? ws + plan.acc_elems : nullptr;
+  a.ws_acc = plan.acc_elems ? ws : nullptr;
+  a.ws_ml = plan.acc_elems ? ws + plan.acc_elems : nullptr;
   a.ws_pref = plan.pref_elems ? reinterpret_cast<int32_t*>(ws + plan.acc_elems + plan.ml_elems)
                               : nullptr;
   a.batch = batch;
@@ -1545,12 +1598,9 @@ int ivakv::decode_append_attn_capped(const char* name, const void* q, const void
                                      float scale, int window, int n_sink, int dtype,
                                      hipStream_t stream, size_t capacity, WorkspaceSource get_ws) {
   if (dtype_size(dtype) == 0) return fail(IVAKV_E_DTYPE, "%s: unknown dtype code %d", name, dtype);
-  const int pp = block_size == kBS && n_sink >= 0
-                     ? single_partition_pages(batch, num_kv_heads, max_blocks, window, n_sink)
-                     : 0;
   Plan plan;
-  const int st = make_plan(name, kFused, batch, num_q_heads, num_kv_heads, head_dim, block_size,
-                           max_blocks, window, n_sink, pp, &plan);
+  const int st = make_decode_plan(name, kFused, batch, num_q_heads, num_kv_heads, head_dim, block_size,
+                                  max_blocks, window, n_sink, dtype_size(dtype), &plan);
   if (st != IVAKV_OK) return st;
   if (plan.ws_bytes > capacity)
     return fail(IVAKV_E_WORKSPACE,
@@ -1563,6 +1613,6 @@ int ivakv::decode_append_attn_capped(const char* name, const void* q, const void
   if (sst != IVAKV_OK) return sst;
   return decode_entry(kFused, name, q, k_pool, v_pool, block_tables, context_lens, out, ws,
                       capacity, batch, num_q_heads, num_kv_heads, head_dim, block_size,
-                      max_blocks, num_pages, scale, window, n_sink, pp, dtype, stream, k_new,
+                      max_blocks, num_pages, scale, window, n_sink, 0, dtype, stream, k_new,
                       v_new);
 }
