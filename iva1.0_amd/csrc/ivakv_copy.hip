@@ -129,6 +129,130 @@ __global__ __launch_bounds__(256) void append_vec_kernel(AppendArgs a) {
   }
 }
 
+// Whole pages of 16-bit rows (16-row pages, head_dim 64 / 128 / 256, 16-byte rows): a wave
+// takes one kv head of 16 tokens that fill one page, so that its V page is written as 16-byte
+// chunks.  What bounds append_vec_kernel on a chunk append is the number of its V stores,
+// eight 2-byte stores per lane and chunk, each of four 32-byte runs; here V's rows pass through
+// LDS and come back transposed (ds_read_b64_tr_b16: lane i of 16 gets column i of four rows).
+//
+// Which tokens fill a page is found per window of 16 tokens, from the slots of the windows
+// around it: a run starts at a token whose slot opens a page and whose 15 successors have the
+// next slots.  Runs never overlap, so at most one starts in a window and belongs to it
+// (running into the next); tokens of no run (a chunk's ends, decode tokens, scattered or
+// repeated slots) are stored element by element by their own window.  Every row load of a wave
+// is issued before its first store; windows x kv heads go in XCD-contiguous order, one head
+// per wave (two: 15.0 against 12.0 us on the ragged chunks below).
+//
+// us against append_vec_kernel, 8 heads x 128 dims from HBM: 11 ragged chunks (4658 rows) 12.0 :
+// 16.7, 8 chunks of 4096 53.7 : 64.9, 16 of 512 15.1 : 14.7, starting mid-page 17.4 : 18.3, 300
+// of 20 18.6 : 22.2; 32 heads, 16 chunks of 512 mid-page 52 : 84; 16 heads x 64, 16 of 512 14.3 :
+// 15.6.  Chosen from kRunTokens rows and kRunElems elements of K up: below, a window's one wave
+// per head is a long chain (512 rows of 8 heads 4.7 : 3.4, 2048 6.3 : 7.6; a decode step of 1024
+// scattered rows 13.2 : 11.0); head_dim 256 from four times that (300 x 20 rows 21.3 : 20.4, 16
+// chunks of 512 13.6 : 17.7).  Rows scattered singly gain nothing (8192 of them 67.9 : 66.7).
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+constexpr int kRunTokens = 2048;
+constexpr int64_t kRunElems = 1 << 21;
+
+template <int D>
+__global__ __launch_bounds__(256) void append_runs_kernel(AppendArgs a) {
+  constexpr int NCH = D / 8;       // 16-byte chunks of a row
+  constexpr int NL = NCH / 4;      // loads per lane of 16 rows
+  constexpr int kRow = D + 16;     // LDS row in elements (32 bytes of padding spread the rows)
+  __shared__ __attribute__((aligned(16))) uint16_t s_v[4][16 * kRow];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int groups = cdiv(a.Hkv, 4);
+  const int64_t blk = xcd_contiguous_block(blockIdx.x, gridDim.x);
+  const int64_t g = blk / groups;
+  const int h = (int)(blk - g * groups) * 4 + wave;
+  if (h >= a.Hkv) return;
+
+  // Slots of tokens 16 g - 16 .. 16 g + 47, one per lane; the window is lanes 16 .. 31.
+  const int64_t tl = 16 * g - 16 + lane;
+  const int64_t slot = tl >= 0 && tl < a.n_tok ? (int64_t)a.slots[tl] : -1;
+  const bool valid = slot >= 0 && slot < a.n_slots;
+  const int next = __shfl_down((int)slot, 1);
+  uint64_t run = __ballot(valid && lane < 63 && next == (int)slot + 1);
+  run &= run >> 1;
+  run &= run >> 2;
+  run &= run >> 4;
+  run &= run >> 7;  // lanes whose next 15 tokens have the next 15 slots
+  const uint64_t starts = run & __ballot(valid && (slot & 15) == 0);
+  const uint64_t own = starts & 0xFFFF0000u, before = starts & 0xFFFFu;
+  uint64_t left = __ballot(valid) & 0xFFFF0000u;
+  if (before) left &= ~(0xFFFFull << __builtin_ctzll(before));
+  if (own) left &= ~(0xFFFFull << __builtin_ctzll(own));
+
+  const uint16_t* kn = static_cast<const uint16_t*>(a.k_new) + h * a.khs;
+  const uint16_t* vn = static_cast<const uint16_t*>(a.v_new) + h * a.vhs;
+  uint16_t* kp = static_cast<uint16_t*>(a.k_pool);
+  uint16_t* vp = static_cast<uint16_t*>(a.v_pool);
+  // The leftover tokens of this window: token lane % 16, chunks 4 i + lane / 16.
+  const int t_lo = lane & 15, c_lo = lane >> 4;
+  const int64_t s_left = __shfl((int)slot, 16 + t_lo);
+  const bool is_left = ((left >> (16 + t_lo)) & 1) != 0;
+  union Row {
+    Chunk16 c16;
+    uint16_t e[8];
+  };
+  Row lk[NL], lv[NL];
+  auto load_left = [&]() {
+    const int64_t t = 16 * g + t_lo;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      lk[i].c16 = load_nt<Chunk16>(kn + t * a.kts + 8 * (4 * i + c_lo));
+      lv[i].c16 = load_nt<Chunk16>(vn + t * a.vts + 8 * (4 * i + c_lo));
+    }
+  };
+  if (own) {
+    const int l0 = __builtin_ctzll(own);
+    const int64_t t0 = 16 * g - 16 + l0;
+    const int64_t page = (int64_t)__shfl((int)slot, l0) >> 4;
+    Chunk16 k[NL], v[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      // K: lanes along the tokens of a chunk, as its page lies; V: along a token's row.
+      k[i] = load_nt<Chunk16>(kn + (t0 + t_lo) * a.kts + 8 * (4 * i + c_lo));
+      v[i] = load_nt<Chunk16>(vn + (t0 + (64 * i + lane) / NCH) * a.vts + 8 * ((64 * i + lane) % NCH));
+    }
+    if (is_left) load_left();
+    const int64_t tile = (page * a.Hkv + h) * (16 * D);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      *reinterpret_cast<Chunk16*>(&s_v[wave][(64 * i + lane) / NCH * kRow + 8 * ((64 * i + lane) % NCH)]) = v[i];
+      store_nt(kp + tile + 8 * (64 * i + lane), k[i]);
+    }
+    __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses take effect in order)
+    // Chunk (dim, half): the 8 tokens 8 half .. of a dim, from two transposed reads of
+    // four rows by 16 dims.
+    const int half = c_lo & 1;
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) {
+      typedef __attribute__((address_space(3))) i16x4_t lds_i16x4;
+      const int d0 = 32 * i + 16 * (lane >> 5);
+      const uint16_t* src = &s_v[wave][(8 * half + (t_lo >> 2)) * kRow + d0 + 4 * (t_lo & 3)];
+      const uint64_t lo = __builtin_bit_cast(uint64_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)src));
+      const uint64_t hi =
+          __builtin_bit_cast(uint64_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 4 * kRow)));
+      const Chunk16 o{{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)}};
+      store_nt(vp + tile + (d0 + t_lo) * 16 + 8 * half, o);
+    }
+  } else if (is_left) {
+    load_left();
+  }
+  if (is_left) {
+    const int row = (int)s_left & 15;
+    const int64_t tile = ((s_left >> 4) * a.Hkv + h) * (16 * D);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int c = 4 * i + c_lo;
+      store_nt(kp + tile + (16 * c + row) * 8, lk[i].c16);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vp[tile + (8 * c + e) * 16 + row] = lv[i].e[e];
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // gather: pages -> k_out / v_out = [B][Hkv][out_len][D]
 // ---------------------------------------------------------------------------
@@ -390,6 +514,18 @@ extern "C" int ivakv_append(const void* k_new, const void* v_new, int64_t k_tok_
   const int threads = few ? 64 : 256;
   const unsigned grid = blocks_for(total, threads);
   if ((int64_t)grid > kMaxGrid) return fail(IVAKV_E_SHAPE, "ivakv_append: too many rows");
+  const int64_t elems = (int64_t)n_tok * num_kv_heads * head_dim;
+  const int scale = head_dim == 256 ? 4 : 1;
+  if (es == 2 && vec && block_size == 16 && (head_dim == 64 || head_dim == 128 || head_dim == 256) &&
+      n_tok >= scale * kRunTokens && elems >= scale * kRunElems) {
+    const int64_t wgs = (int64_t)cdiv(n_tok, 16) * cdiv(num_kv_heads, 4);
+    if (wgs > kMaxGrid) return fail(IVAKV_E_SHAPE, "ivakv_append: too many rows");
+    const dim3 rg((unsigned)wgs);
+    if (head_dim == 64) append_runs_kernel<64><<<rg, 256, 0, stream>>>(a);
+    else if (head_dim == 128) append_runs_kernel<128><<<rg, 256, 0, stream>>>(a);
+    else append_runs_kernel<256><<<rg, 256, 0, stream>>>(a);
+    return launch_status("ivakv_append");
+  }
   if (es == 4) {
     if (few) append_vec_kernel<uint32_t, 1><<<grid, threads, 0, stream>>>(a);
     else if (vec) append_vec_kernel<uint32_t, kAppendHeads><<<grid, threads, 0, stream>>>(a);
