@@ -61,8 +61,12 @@ struct PrefillArgs {
 // two 16-row blocks (two waves per SIMD, under 256 registers each, so one
 // wave's softmax overlaps the other's MFMAs) and two pairs in flight in
 // registers; fp32 and head_dim 256: 4 waves (one per SIMD, the accumulator in
-// AGPRs) and one pair in flight.
-template <int DT, int D>
+// AGPRs) and one pair in flight.  The single launch at head_dim 64 (kSplit false) keeps one
+// pair in flight too and stays under 128 registers, so that two workgroups share a CU and
+// hide each other's barriers and loads: its walks are short (16 x 512 rows of 16 heads 37.1
+// -> 28.7 us, 16 chunks of <= 300 at <= 1000 keys 46.5 -> 39.6).  The split path's
+// persistent workgroups are one per CU and keep the pipeline (93.4 against 95.5 us).
+template <int DT, int D, bool kSplit>
 struct PrefillShape {
   static constexpr int kESize = DT == IVAKV_F32 ? 4 : 2;
   static constexpr int kWaves = (DT == IVAKV_F32 || D == 256) ? 4 : 8;
@@ -70,7 +74,9 @@ struct PrefillShape {
   // Row blocks per wave; one for fp32 at head_dim 256, whose q rows and accumulators
   // for two blocks would not fit 512 registers.
   static constexpr int NR = (DT == IVAKV_F32 && D == 256) ? 1 : 2;
-  static constexpr int kStages = kWaves == 8 ? 2 : 1;  // pairs in flight in registers
+  static constexpr int kStages = kWaves == 8 && (kSplit || D != 64) ? 2 : 1;  // pairs in flight in registers
+  // Waves per SIMD the registers have to allow.
+  static constexpr int kMinWaves = kStages == 1 && kWaves == 8 ? 4 : 1;
   static constexpr int kRowsWave = 16 * NR;
   static constexpr int kRowsWG = kRowsWave * kWaves;
   static constexpr int kPageElems = kBS * D;          // one K or V page tile
@@ -125,13 +131,13 @@ __device__ inline RowBlock row_block(const PrefillArgs& a, const int32_t* ctx, c
 // into partial slot `slot` of the split workspace, for merge_rows.  Every
 // thread of the workgroup calls it with the same arguments (the returns and barriers
 // inside are uniform).
-template <int DT, int D, bool kFp8>
+template <int DT, int D, bool kFp8, bool kSplit>
 __device__ __attribute__((always_inline)) inline void prefill_rows(
     const PrefillArgs& a, const int32_t* __restrict__ bt, const int32_t* __restrict__ ctx,
     const int32_t* __restrict__ qstart, int b, int h, int xb, int pair_lo, int pair_hi, int slot) {
   using Tr = Traits<DT>;
   using E = typename Tr::E;
-  using S = PrefillShape<DT, D>;
+  using S = PrefillShape<DT, D, kSplit>;
   constexpr int X = 16 / (int)sizeof(E);
   constexpr int KLD = D / X / 4;  // 16-byte K reads per lane per page
   constexpr int NB = D / 16;      // 16-dim blocks
@@ -690,7 +696,8 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
 // last first: later rows see more keys, so the longest blocks are dispatched first
 // and the shortest fill the tail.
 template <int DT, int D, bool kFp8>
-__global__ __launch_bounds__((PrefillShape<DT, D>::kThreads)) void prefill_kernel(PrefillArgs a,
+__global__ __launch_bounds__((PrefillShape<DT, D, false>::kThreads), (kFp8 ? 1 : PrefillShape<DT, D, false>::kMinWaves))
+void prefill_kernel(PrefillArgs a,
                                                              const int32_t* __restrict__ bt,
                                                              const int32_t* __restrict__ ctx,
                                                              const int32_t* __restrict__ qstart) {
@@ -699,7 +706,7 @@ __global__ __launch_bounds__((PrefillShape<DT, D>::kThreads)) void prefill_kerne
   if (unit >= a.batch * a.Hkv) return;
   const int b = unit / a.Hkv, h = unit % a.Hkv;
   const int xb = a.blocks_x - 1 - slot % a.blocks_x;
-  prefill_rows<DT, D, kFp8>(a, bt, ctx, qstart, b, h, xb, 0, 0x7fffffff, -1);
+  prefill_rows<DT, D, kFp8, false>(a, bt, ctx, qstart, b, h, xb, 0, 0x7fffffff, -1);
 }
 
 // ---------------------------------------------------------------------------
@@ -993,10 +1000,10 @@ __device__ inline void merge_rows(const PrefillArgs& a, const SplitWs& ws, const
 // dispatcher deals workgroup ids round-robin to the XCDs, so a unit's row blocks and
 // segments share one L2), taking tickets from the queue's counter until it is empty.
 template <int DT, int D, bool kFp8>
-__global__ __launch_bounds__((PrefillShape<DT, D>::kThreads)) void prefill_split_kernel(
+__global__ __launch_bounds__((PrefillShape<DT, D, true>::kThreads)) void prefill_split_kernel(
     PrefillArgs a, const int32_t* __restrict__ bt, const int32_t* __restrict__ ctx,
     const int32_t* __restrict__ qstart, SplitWs ws) {
-  using S = PrefillShape<DT, D>;
+  using S = PrefillShape<DT, D, true>;
   __shared__ int s_ticket[2];
   __shared__ int s_last;
   const int x = blockIdx.x & 7;
@@ -1018,11 +1025,11 @@ __global__ __launch_bounds__((PrefillShape<DT, D>::kThreads)) void prefill_split
     const int2 rb = ws.rb[b * a.blocks_x + xb];
     if (s >= rb.y) continue;  // the block has no rows, or fewer segments
     if (rb.y == 1) {
-      prefill_rows<DT, D, kFp8>(a, bt, ctx, qstart, b, h, xb, 0, 0x7fffffff, -1);
+      prefill_rows<DT, D, kFp8, true>(a, bt, ctx, qstart, b, h, xb, 0, 0x7fffffff, -1);
       continue;
     }
-    prefill_rows<DT, D, kFp8>(a, bt, ctx, qstart, b, h, xb, s * seg, (s + 1) * seg,
-                              rb.x + h * rb.y + s);
+    prefill_rows<DT, D, kFp8, true>(a, bt, ctx, qstart, b, h, xb, s * seg, (s + 1) * seg,
+                                    rb.x + h * rb.y + s);
     // Count the segment in: every wave waits until its partial stores have reached this
     // XCD's L2 (the barrier alone waits only for LDS traffic), then thread 0's
     // agent-scope release writes them back where the other XCDs read, and the arrival
@@ -1057,9 +1064,10 @@ void launch_prefill_d(dim3 grid, hipStream_t stream, const PrefillArgs& a, const
   // LDS beyond 64 KiB (fp32 with head_dim 256) must be allowed per kernel once.
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void*>(&prefill_kernel<DT, D, kFp8>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, (int)PrefillShape<DT, D>::kLdsBytes);
+      hipFuncAttributeMaxDynamicSharedMemorySize, (int)PrefillShape<DT, D, false>::kLdsBytes);
   (void)attr;
-  prefill_kernel<DT, D, kFp8><<<grid, PrefillShape<DT, D>::kThreads, PrefillShape<DT, D>::kLdsBytes, stream>>>(a, bt, ctx, qs);
+  using S = PrefillShape<DT, D, false>;
+  prefill_kernel<DT, D, kFp8><<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, bt, ctx, qs);
 }
 
 template <int DT, bool kFp8 = false>
@@ -1077,7 +1085,7 @@ void launch_prefill(int head_dim, dim3 grid, hipStream_t stream, const PrefillAr
 template <int DT, int D, bool kFp8>
 void launch_split_d(int n_wg, hipStream_t stream, const PrefillArgs& a, const int32_t* bt,
                     const int32_t* ctx, const int32_t* qs, const SplitWs& ws) {
-  using S = PrefillShape<DT, D>;
+  using S = PrefillShape<DT, D, true>;
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void*>(&prefill_split_kernel<DT, D, kFp8>),
       hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kLdsBytes);
@@ -1109,9 +1117,9 @@ int split_workgroups() {
 template <int DT>
 int rows_per_workgroup_t(int head_dim) {
   switch (head_dim) {
-    case 64: return PrefillShape<DT, 64>::kRowsWG;
-    case 128: return PrefillShape<DT, 128>::kRowsWG;
-    default: return PrefillShape<DT, 256>::kRowsWG;
+    case 64: return PrefillShape<DT, 64, true>::kRowsWG;
+    case 128: return PrefillShape<DT, 128, true>::kRowsWG;
+    default: return PrefillShape<DT, 256, true>::kRowsWG;
   }
 }
 
