@@ -166,6 +166,10 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const Chunk16* up, const Ch
 
 constexpr int kLinearBlocks = 4;  // blocks of 64 k in one load set of a wave
 
+// How linear_rows normalizes its rows: not, into LDS before the products, or by scaling the
+// sums after them.
+enum Norm { kNoNorm = 0, kNormLds = 1, kNormFold = 2 };
+
 enum Epilogue { kPlain = 0, kResidual = 1, kSwiglu = 2 };
 
 struct LinearArgs {
@@ -193,22 +197,30 @@ struct LinearArgs {
 // registers for all its tiles and the next tile's weights are loaded before this tile's
 // sums meet.  Otherwise the sets alternate along k and x is read again (L2) per tile.
 //
-// NORM (MT 1): x is RMS-normalized first, each workgroup for itself (the rows are L2 hits),
-// into LDS rows of k + 8 elements (the pad spreads the rows over the banks); the wave's
-// first weight loads are issued before that and arrive meanwhile.
+// NORM (MT 1): x is RMS-normalized, each workgroup for itself (the rows are L2 hits).
+//   kNormLds   into LDS rows of k + 8 elements (the pad spreads the rows over the banks), the
+//              wave's first weight loads issued before that.
+//   kNormFold  (bf16) the products take x * norm_w, rounded once, and the sums are scaled by
+//              the rows' 1 / rms at the end; each wave sums the squares of its part of k, so
+//              nothing waits for whole rows.  16 rows: q / k / v 7.0 -> 5.5 us, gate / up 9.0 ->
+//              7.1; one row 4.3 -> 4.8 and 6.0 -> 6.6, so up to kNormLdsRows rows stay with LDS.
+//              In fp16 the product could overflow where the normalized row does not.
 //
 // 16 rows, bf16, weights from HBM, against the library's products (us): q / k / v (3 x 1024
-// x 1024) 4.6, with the norm 7.0, against 3 x 5.6; 1024 x 1024 with residual 4.0 against
-// 5.6 + 2.4; gate / up (2 x 4096 x 1024) with norm and SwiGLU 9.0 against 2 x 7.6 + 5.2 + 21;
+// x 1024) 4.6, with the norm 5.5, against 3 x 5.6; 1024 x 1024 with residual 4.0 against
+// 5.6 + 2.4; gate / up (2 x 4096 x 1024) with norm and SwiGLU 7.1 against 2 x 7.6 + 5.2 + 21;
 // 1024 x 4096 10.3 against 14.4 (64 column tiles reach 64 CUs, whose loads bound it: 7.6 at
 // one row); 32000 x 1024 18.3 against 19.3.
-template <int DT, int MT, int WAVES, bool NORM, int EPI, bool ONE>
+template <int DT, int MT, int WAVES, int NORM, int EPI, bool ONE>
 __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(LinearArgs a) {
   using Tr = Traits<DT>;
   using E = typename Tr::E;
   constexpr int NT = EPI == kSwiglu ? 2 : 1;
   constexpr int U = kLinearBlocks;
   constexpr int NCN = WAVES / 2;    // norm: 16-byte chunks of a row per lane (k <= 256 WAVES)
+  constexpr bool FOLD = NORM == kNormFold;
+  constexpr bool NORM_LDS = NORM == kNormLds;
+  static_assert(!FOLD || (ONE && MT == 1), "the folded norm keeps its rows in registers");
   extern __shared__ Chunk16 smem[];
   const int lane = threadIdx.x & 63, ln = lane & 15, lq = lane >> 4;
   const int wave = uni(threadIdx.x >> 6);
@@ -247,10 +259,10 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(LinearArgs a) {
       }
     }
   };
-  load_w(0, blockIdx.x, b0);
+  if constexpr (!FOLD) load_w(0, blockIdx.x, b0);
 
   const int xs = k + 8;  // LDS row of the normalized x
-  if constexpr (NORM) {
+  if constexpr (NORM_LDS) {
     E* xn = reinterpret_cast<E*>(smem);
     const int n8 = k >> 3;
     for (int r = wave; r < m; r += WAVES) {
@@ -291,7 +303,7 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(LinearArgs a) {
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int r = min(16 * t + ln, m - 1);  // rows past m repeat the last; never stored
-    xp[t] = NORM ? reinterpret_cast<const E*>(smem) + r * xs + 16 * lq
+    xp[t] = NORM_LDS ? reinterpret_cast<const E*>(smem) + r * xs + 16 * lq
                  : static_cast<const E*>(a.x) + r * a.ldx + 16 * lq;
   }
   f32x4 acc[MT][NT];
@@ -323,10 +335,47 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(LinearArgs a) {
 #pragma unroll
     for (int t = 0; t < MT; ++t) load_x(t, b0);
   }
+  Chunk16 nw[FOLD ? U : 1][2];
+  if constexpr (FOLD) {
+    load_w(0, blockIdx.x, b0);
+    if (a.norm_w) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const E* p = static_cast<const E*>(a.norm_w) + 16 * lq + 64 * min(b0 + u, last);
+        nw[u][0] = *reinterpret_cast<const Chunk16*>(p);
+        nw[u][1] = *reinterpret_cast<const Chunk16*>(p + 8);
+      }
+    }
+  }
 
   // Sums over the waves, in two LDS buffers used in turn (one barrier per tile): tile t of
-  // the rows by wave t.  With NORM they lie behind the normalized rows.
-  f32x4* red0 = reinterpret_cast<f32x4*>(smem) + (NORM ? (m * xs + 7) / 8 : 0);
+  // the rows by wave t.  With NORM they lie behind the normalized rows or the rows' sums of
+  // squares.
+  f32x4* red0 = reinterpret_cast<f32x4*>(smem) + (NORM_LDS ? (m * xs + 7) / 8 : FOLD ? 4 * WAVES : 0);
+  float* s_ss = reinterpret_cast<float*>(smem);  // FOLD: [WAVES][16]
+  if constexpr (FOLD) {
+    float ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float part = 0.f;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const bf16x2 x2 = __builtin_bit_cast(bf16x2, xv[0][u][j].w[i]);
+          part = __builtin_amdgcn_fdot2_f32_bf16(x2, x2, part, false);  // exact products, fp32 sum
+          if (a.norm_w) {
+            const bf16x2 w2 = __builtin_bit_cast(bf16x2, nw[u][j].w[i]);
+            xv[0][u][j].w[i] = Tr::pack2((float)x2[0] * (float)w2[0], (float)x2[1] * (float)w2[1]);
+          }
+        }
+      }
+      ss += b0 + u < b1 ? part : 0.f;
+    }
+    ss += __shfl_xor(ss, 16);
+    ss += __shfl_xor(ss, 32);
+    if (lane < 16) s_ss[wave * 16 + lane] = ss;  // (published by the first sums' barrier)
+  }
   auto finish = [&](int par, int t_flat) IVAKV_INLINE {
     f32x4* red = red0 + par * (MT * NT * WAVES * 64);
 #pragma unroll
@@ -342,6 +391,14 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(LinearArgs a) {
       s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < WAVES; ++u) s[j] += red[((wave * NT + j) * WAVES + u) * 64 + lane];
+    }
+    if constexpr (FOLD) {
+      float ss = 0.f;
+#pragma unroll
+      for (int u = 0; u < WAVES; ++u) ss += s_ss[u * 16 + ln];
+      const float inv = 1.f / sqrtf(ss / (float)k + a.eps);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) s[j] *= inv;
     }
     int seg, tile;
     locate(t_flat, seg, tile);
@@ -403,15 +460,17 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(LinearArgs a) {
 constexpr int kLinearMaxRows = 32;
 constexpr int kLinearNormRows = 16;
 constexpr int kLinearNormMaxK = 2048;
+constexpr int kNormLdsRows = 4;
 
 // Workgroups of a launch: what the CUs hold at once (four of 4 waves, two of 8),
 // each taking tiles a grid apart.
 constexpr int kLinearWaves = 256 * 16;
 
-template <int DT, int MT, int WAVES, bool NORM, int EPI, bool ONE>
+template <int DT, int MT, int WAVES, int NORM, int EPI, bool ONE>
 void launch_linear_one(const LinearArgs& a, hipStream_t stream) {
   size_t smem = (size_t)2 * MT * (EPI == kSwiglu ? 2 : 1) * WAVES * 64 * sizeof(f32x4);
-  if (NORM) smem += ((size_t)a.m * (a.k + 8) + 7) / 8 * 16;
+  if (NORM == kNormLds) smem += ((size_t)a.m * (a.k + 8) + 7) / 8 * 16;
+  if (NORM == kNormFold) smem += (size_t)64 * WAVES;
   // (beyond 64 KiB of LDS must be allowed per kernel once)
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void*>(&linear_rows_kernel<DT, MT, WAVES, NORM, EPI, ONE>),
@@ -421,26 +480,28 @@ void launch_linear_one(const LinearArgs& a, hipStream_t stream) {
   linear_rows_kernel<DT, MT, WAVES, NORM, EPI, ONE><<<dim3((unsigned)wgs), 64 * WAVES, smem, stream>>>(a);
 }
 
-template <int DT, int MT, int WAVES, bool NORM, int EPI>
+template <int DT, int MT, int WAVES, int NORM, int EPI>
 void launch_linear(const LinearArgs& a, hipStream_t stream) {
   if (NORM || (MT == 1 && a.k <= 64 * kLinearBlocks * WAVES))
     launch_linear_one<DT, MT, WAVES, NORM, EPI, MT == 1>(a, stream);
   else
-    launch_linear_one<DT, MT, WAVES, NORM, EPI, NORM>(a, stream);
+    launch_linear_one<DT, MT, WAVES, NORM, EPI, NORM != kNoNorm>(a, stream);
 }
 
-template <int DT, int MT, int WAVES, bool NORM>
+template <int DT, int MT, int WAVES, int NORM>
 void launch_linear_e(const LinearArgs& a, int epi, hipStream_t stream) {
   if (epi == kSwiglu) launch_linear<DT, MT, WAVES, NORM, kSwiglu>(a, stream);
   else if (epi == kPlain) launch_linear<DT, MT, WAVES, NORM, kPlain>(a, stream);
-  else if constexpr (!NORM) launch_linear<DT, MT, WAVES, NORM, kResidual>(a, stream);
+  else if constexpr (NORM == kNoNorm) launch_linear<DT, MT, WAVES, NORM, kResidual>(a, stream);
 }
 
 template <int DT, int WAVES>
 void launch_linear_m(const LinearArgs& a, bool norm, int epi, hipStream_t stream) {
-  if (norm) launch_linear_e<DT, 1, WAVES, true>(a, epi, stream);
-  else if (a.m <= 16) launch_linear_e<DT, 1, WAVES, false>(a, epi, stream);
-  else launch_linear_e<DT, 2, WAVES, false>(a, epi, stream);
+  if (norm && DT == IVAKV_BF16 && a.m > kNormLdsRows)
+    launch_linear_e<DT, 1, WAVES, DT == IVAKV_BF16 ? kNormFold : kNormLds>(a, epi, stream);
+  else if (norm) launch_linear_e<DT, 1, WAVES, kNormLds>(a, epi, stream);
+  else if (a.m <= 16) launch_linear_e<DT, 1, WAVES, kNoNorm>(a, epi, stream);
+  else launch_linear_e<DT, 2, WAVES, kNoNorm>(a, epi, stream);
 }
 
 template <int DT>

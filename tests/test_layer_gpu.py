@@ -64,7 +64,7 @@ def test_swiglu(iva, dev, dtype, n):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("k,n", [(64, 16), (320, 48), (1024, 32), (1088, 16), (2048, 64), (4160, 32)])
-@pytest.mark.parametrize("m", [1, 16, 17, 32])
+@pytest.mark.parametrize("m", [1, 4, 5, 16, 17, 32])
 def test_linear_rows(iva, dev, dtype, m, k, n):
     ops = iva.ops
     x = _randn((m, k), 3, dev, dtype)
@@ -83,11 +83,22 @@ def test_linear_rows(iva, dev, dtype, m, k, n):
           2 * sums * (1 + ug[0].abs() + ug[1].abs()))
     if m <= ops.LINEAR_NORM_MAX_ROWS and k <= ops.LINEAR_NORM_MAX_K:
         nw = _randn(k, 10, dev, dtype)
-        y = ops.rms_norm(x, nw, 1e-6)  # the fused norm rounds as the kernel alone does
-        for got, alone in zip(ops.linear_rows(x, w, norm=(nw, 1e-6)), ops.linear_rows(y, w)):
-            assert torch.equal(got, alone)
-        assert torch.equal(ops.linear_rows(x, [w[0], up], norm=(nw, 1e-6), swiglu_pair=True),
-                           ops.linear_rows(y, [w[0], up], swiglu_pair=True))
+        y = ops.rms_norm(x, nw, 1e-6)
+        fused = ops.linear_rows(x, w, norm=(nw, 1e-6))
+        pair = ops.linear_rows(x, [w[0], up], norm=(nw, 1e-6), swiglu_pair=True)
+        if dtype == torch.float16 or m <= 4:  # normalized as the kernel alone does
+            for got, alone in zip(fused, ops.linear_rows(y, w)):
+                assert torch.equal(got, alone)
+            assert torch.equal(pair, ops.linear_rows(y, [w[0], up], swiglu_pair=True))
+        else:  # x * nw rounded once (u each product), the sums scaled by 1 / rms
+            yd = _norm64(x, nw)
+            for got, wi in zip(fused, w):
+                check(got, yd @ wi.double().t(), 1.01 * U[dtype] * (yd.abs() @ wi.double().abs().t()))
+            e = [1.01 * U[dtype] * (yd.abs() @ t.double().abs().t()) for t in (up, w[0])]
+            u, g = yd @ up.double().t(), yd @ w[0].double().t()
+            # |d silu| <= 1.1 |du|
+            check(pair, F.silu(u) * g, 1.2 * e[0] * (g.abs() + e[1]) + F.silu(u).abs() * e[1]
+                  + 2 * sums * (1 + u.abs() + g.abs()))
 
 
 def test_linear_rows_many_tiles(iva, dev):
