@@ -122,11 +122,13 @@ int ivakv_decode_workspace_size(int batch, int num_q_heads, int num_kv_heads,
  * wavefronts sized to the device; a (sequence, kv head) split between
  * wavefronts is merged with a log-sum-exp reduction.  partition_pages > 0
  * instead splits each sequence into partitions of that many pages (one
- * workgroup each) merged the same way.  With partition_pages <= 0, a batch of one
- * to four (sequence, kv head) units per CU on tables of at most 64 effective pages
- * takes one partition per sequence in a single launch (no merge: the call then
- * accepts a null workspace; ivakv_decode_workspace_size still reports the stream
- * walk's need, which covers it).
+ * workgroup each) merged the same way.  With partition_pages <= 0, a batch of at
+ * least one (sequence, kv head) unit per CU on tables of at most 64 effective
+ * pages, or of fewer units on tables of at most 32 pages and 256 KiB of K and V a
+ * unit, takes one partition per sequence in a single launch with no merge (with
+ * one to four units per CU the call then accepts a null workspace;
+ * ivakv_decode_workspace_size reports the stream walk's need in every case, which
+ * covers it).
  * Supported: block_size 16, head_dim 64/128/256, num_q_heads/num_kv_heads
  * (the GQA group) any integer from 1 to 16.
  * Replaces: the cache branch of AttentionTorch.forward -- scores, causal /

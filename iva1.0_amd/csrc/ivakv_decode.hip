@@ -409,8 +409,8 @@ struct TileOps8 {
 // an invalid page id; every wave's padding reads that tile, an L2 hit, where its own last
 // tile, loaded for streaming, would miss) and the slot is fully masked, so the loop body has
 // no branches and the compiler's vmcnt waits only cover the buffer about to be consumed.  The
-// last round of the ring loads nothing: with it (two more tiles per wave and unit) 256 units
-// of 32 pages took 18.3 us of the 15.7 they take without.
+// last round of the ring loads nothing: two more tiles per wave and unit would be read and
+// masked (512 units of 32 pages 28.4 -> 26.8 us without them, 1024 units 57.2 -> 49.3).
 //
 // Built for two workgroups per CU (one at head_dim 256): with a higher
 // occupancy target the scheduler sinks each load next to its use and the ring

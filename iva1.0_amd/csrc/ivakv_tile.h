@@ -49,15 +49,6 @@ __device__ inline void mask_rows16(Chunk8& v, const bool vis[4]) {
   v.w[1] &= (vis[2] ? 0x0000FFFFu : 0u) | (vis[3] ? 0xFFFF0000u : 0u);
 }
 
-// The same over a page pair's operand: 4 rows of page A (words 0-1), then 4 of
-// page B (words 2-3).
-__device__ inline void mask_pair16(Chunk16& v, const bool va[4], const bool vb[4]) {
-  v.w[0] &= (va[0] ? 0x0000FFFFu : 0u) | (va[1] ? 0xFFFF0000u : 0u);
-  v.w[1] &= (va[2] ? 0x0000FFFFu : 0u) | (va[3] ? 0xFFFF0000u : 0u);
-  v.w[2] &= (vb[0] ? 0x0000FFFFu : 0u) | (vb[1] ? 0xFFFF0000u : 0u);
-  v.w[3] &= (vb[2] ? 0x0000FFFFu : 0u) | (vb[3] ? 0xFFFF0000u : 0u);
-}
-
 template <int DT>
 struct Traits;
 
@@ -91,9 +82,6 @@ struct Traits<IVAKV_F16> {
   static __device__ inline PP8 pack_pp8(const float pa[4], const float pb[4]) { return pack_p8(pa, pb); }
   static __device__ inline f32x4 pv_pair(const VPair& v, const PP8& p, f32x4 acc) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, v), p, acc, 0, 0, 0);
-  }
-  static __device__ inline void mask_pair(VPair& v, const bool va[4], const bool vb[4]) {
-    mask_pair16(v, va, vb);
   }
   static __device__ inline E from_float(float x) { return (E)x; }
   // Two values rounded to E (nearest even), packed low first.
@@ -141,9 +129,6 @@ struct Traits<IVAKV_BF16> {
   }
   static __device__ inline f32x4 pv_pair(const VPair& v, const PP8& p, f32x4 acc) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, v), p, acc, 0, 0, 0);
-  }
-  static __device__ inline void mask_pair(VPair& v, const bool va[4], const bool vb[4]) {
-    mask_pair16(v, va, vb);
   }
   static __device__ inline E from_float(float x) { return (E)x; }
   static __device__ inline uint32_t pack2(float a, float b) {
@@ -195,10 +180,6 @@ struct Traits<IVAKV_F32> {
   static __device__ inline void mask_rows(VChunk& v, const bool vis[4]) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) v.w[r] = vis[r] ? v.w[r] : 0u;
-  }
-  static __device__ inline void mask_pair(VPair& v, const bool va[4], const bool vb[4]) {
-    mask_rows(v.a, va);
-    mask_rows(v.b, vb);
   }
 };
 
