@@ -487,7 +487,8 @@ int ivakv_swiglu(const void* up, const void* gate, void* out, int64_t n, int dty
  * to three matrices (n1, n2 may be 0) in one launch, each streamed once.  m <= 32, k a
  * multiple of 64, n_i of 16, ldx (the row stride of x, >= k) of 8.
  *   norm != 0     x is RMS-normalized first, as ivakv_rms_norm does (norm_weight may be
- *                 null); m <= 16, k <= 2048, epilogue 0 or 2.
+ *                 null; bf16 may round x * weight and scale the fp32 sums by 1 / rms
+ *                 instead); m <= 16, k <= 2048, epilogue 0 or 2.
  *   epilogue 1    out0 += residual[m][n0]  (one matrix)
  *   epilogue 2    out0 = silu(x w1^T) * (x w0^T): w0 the gate, w1 the up projection
  *                 (n1 == n0, out1 unused)
