@@ -6,6 +6,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <atomic>
+
 #include "ivakv.h"
 
 namespace ivakv {
@@ -75,6 +77,17 @@ template <bool NT, class T>
 __device__ inline void st(void* p, const T& v) {
   if constexpr (NT) store_nt<T>(p, v);
   else *static_cast<T*>(p) = v;
+}
+
+// Allows `kernel` `bytes` of dynamic LDS, which has to be asked for above 64 KiB, once per
+// device (`done`: bits of the devices asked, kept by the caller for this kernel).
+inline void allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
+  int dev = 0;
+  if (bytes <= 64 * 1024 || hipGetDevice(&dev) != hipSuccess) return;
+  const uint64_t bit = dev < 64 ? 1ull << dev : 0;
+  if (done.load(std::memory_order_relaxed) & bit) return;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess)
+    done.fetch_or(bit, std::memory_order_relaxed);
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

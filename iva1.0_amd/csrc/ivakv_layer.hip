@@ -471,11 +471,11 @@ void launch_linear_one(const LinearArgs& a, hipStream_t stream) {
   size_t smem = (size_t)2 * MT * (EPI == kSwiglu ? 2 : 1) * WAVES * 64 * sizeof(f32x4);
   if (NORM == kNormLds) smem += ((size_t)a.m * (a.k + 8) + 7) / 8 * 16;
   if (NORM == kNormFold) smem += (size_t)64 * WAVES;
-  // (beyond 64 KiB of LDS must be allowed per kernel once)
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&linear_rows_kernel<DT, MT, WAVES, NORM, EPI, ONE>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  (void)attr;
+  if (smem > 64 * 1024) {  // (the size depends on m and k: the whole LDS is asked for)
+    static std::atomic<uint64_t> done{0};
+    allow_lds(reinterpret_cast<const void*>(&linear_rows_kernel<DT, MT, WAVES, NORM, EPI, ONE>),
+              160 * 1024, done);
+  }
   const int wgs = a.tiles < kLinearWaves / WAVES ? a.tiles : kLinearWaves / WAVES;
   linear_rows_kernel<DT, MT, WAVES, NORM, EPI, ONE><<<dim3((unsigned)wgs), 64 * WAVES, smem, stream>>>(a);
 }

@@ -1061,12 +1061,9 @@ __global__ __launch_bounds__((PrefillShape<DT, D, true>::kThreads)) void prefill
 template <int DT, int D, bool kFp8>
 void launch_prefill_d(dim3 grid, hipStream_t stream, const PrefillArgs& a, const int32_t* bt,
                       const int32_t* ctx, const int32_t* qs) {
-  // LDS beyond 64 KiB (fp32 with head_dim 256) must be allowed per kernel once.
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&prefill_kernel<DT, D, kFp8>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, (int)PrefillShape<DT, D, false>::kLdsBytes);
-  (void)attr;
   using S = PrefillShape<DT, D, false>;
+  static std::atomic<uint64_t> done{0};
+  allow_lds(reinterpret_cast<const void*>(&prefill_kernel<DT, D, kFp8>), (int)S::kLdsBytes, done);
   prefill_kernel<DT, D, kFp8><<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, bt, ctx, qs);
 }
 
@@ -1086,10 +1083,8 @@ template <int DT, int D, bool kFp8>
 void launch_split_d(int n_wg, hipStream_t stream, const PrefillArgs& a, const int32_t* bt,
                     const int32_t* ctx, const int32_t* qs, const SplitWs& ws) {
   using S = PrefillShape<DT, D, true>;
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&prefill_split_kernel<DT, D, kFp8>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kLdsBytes);
-  (void)attr;
+  static std::atomic<uint64_t> done{0};
+  allow_lds(reinterpret_cast<const void*>(&prefill_split_kernel<DT, D, kFp8>), (int)S::kLdsBytes, done);
   prefill_plan_kernel<<<1, kPlanThreads, 0, stream>>>(a, ctx, qs, ws, S::kRowsWG, n_wg);
   prefill_split_kernel<DT, D, kFp8><<<n_wg, S::kThreads, S::kLdsBytes, stream>>>(a, bt, ctx, qs, ws);
 }
