@@ -205,7 +205,8 @@ class LayeredKVCache:
 
 def _plain_mode() -> bool:
     """No grad, autocast, trace, compile, functorch level, forward-mode level, torch
-    function or dispatch mode is active."""
+    function or dispatch mode is active.  Asked before anything of a tensor is looked at:
+    under a functorch transform a tensor has no address to look at."""
     return not (torch.is_grad_enabled() or torch._C._len_torch_function_stack()
                 or torch._C._len_torch_dispatch_stack() or torch.is_autocast_enabled("cuda")
                 or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
@@ -622,7 +623,7 @@ class RMSNorm(nn.Module):
                 and (w is None or (_plain_weight(w, x) and tuple(w.shape) == x.shape[-1:])))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if _plain_input(x) and _plain_mode() and self._kernel_takes(x):
+        if _plain_mode() and _plain_input(x) and self._kernel_takes(x):
             return rms_norm(x, self.weight, self.eps)
         xf = x.float()
         y = xf / torch.sqrt(torch.mean(xf * xf, dim=-1, keepdim=True) + self.eps)
@@ -661,7 +662,7 @@ class FFN(nn.Module):
                 if w is not None:
                     return linear_rows(linear_rows(x, w[:2], swiglu_pair=True), w[2:])
             up, gate = self.up_proj(x), self.gate_proj(x)
-            if (_plain_input(up) and _plain_mode() and _plain_weight(gate, up)
+            if (_plain_mode() and _plain_input(up) and _plain_weight(gate, up)
                     and gate.shape == up.shape and up.numel() % 8 == 0):
                 hidden = swiglu(up, gate)
             else:
