@@ -206,10 +206,12 @@ class LayeredKVCache:
 def _plain_mode() -> bool:
     """No grad, autocast, trace, compile, functorch level, forward-mode level, torch
     function or dispatch mode is active.  Asked before anything of a tensor is looked at:
-    under a functorch transform a tensor has no address to look at."""
-    return not (torch.is_grad_enabled() or torch._C._len_torch_function_stack()
-                or torch._C._len_torch_dispatch_stack() or torch.is_autocast_enabled("cuda")
-                or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+    under a functorch transform a tensor has no address to look at.  Compilation is asked
+    first of all: the compiler takes that as a constant and follows nothing of the rest."""
+    return not (torch.compiler.is_compiling() or torch.is_grad_enabled()
+                or torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack()
+                or torch.is_autocast_enabled("cuda")
+                or torch._C._get_tracing_state() is not None
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or fwAD._current_level >= 0)
 
@@ -623,8 +625,9 @@ class RMSNorm(nn.Module):
                 and (w is None or (_plain_weight(w, x) and tuple(w.shape) == x.shape[-1:])))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if _plain_mode() and _plain_input(x) and self._kernel_takes(x):
-            return rms_norm(x, self.weight, self.eps)
+        if not torch.jit.is_scripting():  # (what is inside is not scripted)
+            if _plain_mode() and _plain_input(x) and self._kernel_takes(x):
+                return rms_norm(x, self.weight, self.eps)
         xf = x.float()
         y = xf / torch.sqrt(torch.mean(xf * xf, dim=-1, keepdim=True) + self.eps)
         y = y.to(x.dtype)

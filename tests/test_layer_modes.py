@@ -37,3 +37,39 @@ def test_functorch_transforms_of_16bit_gpu_tensors(iva, monkeypatch, name, trans
         got = TRANSFORMS[transform](f, x)
         monkeypatch.undo()
     assert torch.equal(got, ref)
+
+
+def _compiled(model, name, x, grad):
+    f = _module(model, name) if name != "model" else lambda ids: model(ids)["logits"]
+    with torch.set_grad_enabled(grad):
+        torch._dynamo.reset()
+        return torch.compile(f, backend="eager", fullgraph=True)(x), f(x)
+
+
+@pytest.mark.parametrize("name", ["norm", "ffn", "block", "model"])
+@pytest.mark.parametrize("grad", [False, True])
+def test_compiles_in_one_graph(iva, name, grad):
+    x = torch.randint(0, 64, (2, 4)) if name == "model" else torch.randn(2, 4, 64)
+    got, ref = _compiled(_model(iva), name, x, grad)
+    assert torch.equal(got, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["norm", "ffn", "block", "model"])
+@pytest.mark.parametrize("grad", [False, True])
+def test_compiles_in_one_graph_16bit(iva, dev, name, grad):
+    """The graph holds the torch operators; without grad the plain call runs the layer kernels."""
+    model = _model(iva, torch.bfloat16).to(dev)
+    x = (torch.randint(0, 64, (2, 4), device=dev) if name == "model"
+         else torch.randn(2, 4, 64, device=dev, dtype=torch.bfloat16))
+    got, ref = _compiled(model, name, x, grad)
+    # (norm: the torch operators round twice, as the kernel; a block rounds six times in a row)
+    assert (got - ref).float().norm() <= 6 * 2.0 ** -8 * ref.float().norm()
+
+
+@pytest.mark.parametrize("affine", [False, True])
+def test_norm_scripts(iva, affine):
+    cfg = iva.TransformerConfig(d_model=64, n_heads=2, n_layers=1, vocab_size=64, elementwise_affine=affine)
+    norm, x = iva.model.RMSNorm(cfg), torch.randn(3, 64)
+    with torch.no_grad():
+        assert torch.equal(torch.jit.script(norm)(x), norm(x))
