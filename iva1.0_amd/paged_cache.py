@@ -377,8 +377,8 @@ class PagedKVPool:
 
 
 class _Slots:
-    """The slot mapping of a forward's new tokens, computed on the device when first needed
-    (the fused decode step finds its slots itself)."""
+    """The slot mapping of a forward's new tokens, computed on the tables' device when first
+    needed (the fused decode step finds its slots itself)."""
 
     def __init__(self, block_tables, context_lens, n: int, block_size: int):
         self._args = (block_tables, context_lens, n, block_size)
@@ -386,7 +386,12 @@ class _Slots:
 
     def get(self) -> torch.Tensor:
         if self._slots is None:
-            self._slots = chunk_slots(*self._args)
+            tables, lens, n, bs = self._args
+            if tables.is_cuda:
+                self._slots = chunk_slots(*self._args)
+            else:  # a cache kept on the host (the kernels run on the GPU only)
+                pos = (lens.view(-1, 1) - n + torch.arange(n, dtype=torch.int32)).long()
+                self._slots = (tables.gather(1, pos // bs) * bs + pos % bs).to(torch.int32).view(-1)
         return self._slots
 
 

@@ -326,3 +326,18 @@ def test_cache_window_policy_releases_and_guards(iva):
     keep.note_window(None)                      # nothing was released: any window is fine
     c2 = pc.create_kv_cache(2, 2, 64, 0, "cpu", pool=p)
     assert isinstance(c2, pc.PagedKVCache) and c2.seq_len == 0 and c2.batch_size == 2
+
+
+def test_slots_of_a_cache_kept_on_the_host(iva):
+    """A forward's slot mapping without a GPU: the allocator's slots of its new tokens."""
+    import torch
+    cache = iva.PagedKVCache(3, 2, 64, 0, "cpu", torch.float16, num_layers=2, max_seq_len=64)
+    for t in (5, 0, 17, 1):
+        rows = torch.zeros(3, t, 2, 64, dtype=torch.float16)
+        start = cache.seq_len
+        for _ in range(2):
+            view = cache.layer_step(rows, rows, append=False)
+            want = [cache.pool.slots(s, np.arange(start, start + t)) for s in cache.seq_ids]
+            assert view.slot_mapping.dtype == torch.int32
+            assert view.slot_mapping.tolist() == np.concatenate(want).tolist()
+            assert view.context_lens.tolist() == [start + t] * 3
