@@ -253,16 +253,14 @@ def decode_workspace_bytes(batch: int, num_q_heads: int, num_kv_heads: int, head
                            partition_pages: int = 0) -> int:
     """Workspace bytes :func:`paged_decode_attention` needs (0 when no sequence spans more
     than one partition).  The workspace needs no initialisation."""
-    return _decode_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, block_size,
-                                   max_blocks, window, n_sink, partition_pages)
-
-
-@lru_cache(maxsize=1024)
-def _decode_workspace_bytes(*geometry) -> int:
-    """A function of the geometry alone (the plan's sizes)."""
     out = ctypes.c_size_t(0)
-    _abi.call("ivakv_decode_workspace_size", *geometry, ctypes.byref(out))
+    _abi.call("ivakv_decode_workspace_size", batch, num_q_heads, num_kv_heads, head_dim,
+              block_size, max_blocks, window, n_sink, partition_pages, ctypes.byref(out))
     return int(out.value)
+
+
+# The ops' own calls, whose arguments are plain integers: a function of the geometry alone.
+_decode_workspace_bytes = lru_cache(maxsize=1024)(decode_workspace_bytes)
 
 
 # Split prefill (ivakv_prefill_attn_split) by default, up to the split path's largest
@@ -370,8 +368,8 @@ def _decode(entry: str, q, k_pool, v_pool, block_tables, context_lens, scale, wi
         if out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
             raise ValueError("out must be a contiguous tensor shaped and typed like q")
         _buffer(out, dev, "out")
-    nbytes = decode_workspace_bytes(batch, hq, hkv, head_dim, bs, max_blocks, window, n_sink,
-                                    partition_pages)
+    nbytes = _decode_workspace_bytes(batch, hq, hkv, head_dim, bs, max_blocks, window, n_sink,
+                                     partition_pages)
     if workspace is None:
         workspace = _workspace(dev, nbytes)
     else:
@@ -492,7 +490,7 @@ def paged_decode_append_attention(q: torch.Tensor, k_new: torch.Tensor, v_new: t
         if out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
             raise ValueError("out must be a contiguous tensor shaped and typed like q")
         _buffer(out, dev, "out")
-    nbytes = decode_workspace_bytes(batch, hq, hkv, head_dim, bs, max_blocks, window, n_sink)
+    nbytes = _decode_workspace_bytes(batch, hq, hkv, head_dim, bs, max_blocks, window, n_sink)
     if workspace is None:
         workspace = _workspace(dev, nbytes)
     else:
@@ -809,8 +807,8 @@ def block_decode(x: torch.Tensor, norm1, eps1: float, wq, wk, wv, wo, norm2, eps
         _scales(k_pool, k_scale, v_scale)
     hidden, max_blocks = wup.shape[0], block_tables.shape[1]
     out = torch.empty_like(x)
-    ws = _workspace(dev, decode_workspace_bytes(m, num_q_heads, hkv, head_dim, bs, max_blocks, window,
-                                                n_sink))
+    ws = _workspace(dev, _decode_workspace_bytes(m, num_q_heads, hkv, head_dim, bs, max_blocks, window,
+                                                 n_sink))
     nbytes = 2 * m * (3 * d + 2 * (num_q_heads + hkv) * head_dim + hidden) + 7 * 256
     scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     args = _abi.BLOCK_DECODE.pack(

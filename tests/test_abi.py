@@ -97,6 +97,19 @@ def test_decode_argument_checks(iva):
         assert call(iva, entry, *decode_args(iva, bs=8)) == a.E_SHAPE
 
 
+def test_workspace_size_is_asked_anew(iva):
+    """The public query keeps no answer by an argument's identity or by its being equal to
+    an earlier one of another type."""
+    import ctypes
+    import torch
+    ws, batch = iva.decode_workspace_bytes, torch.tensor(2)
+    two = ws(2, 32, 8, 128, 16, 100)
+    assert ws(batch, 32, 8, 128, 16, 100) == two
+    assert ws(batch.fill_(9), 32, 8, 128, 16, 100) == ws(9, 32, 8, 128, 16, 100) > two
+    with pytest.raises(ctypes.ArgumentError):
+        ws(2.0, 32, 8, 128, 16, 100)
+
+
 def test_workspace_size(iva):
     ws = iva.decode_workspace_bytes
     # explicit partitions, one per sequence: no workspace
