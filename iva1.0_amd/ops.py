@@ -805,6 +805,7 @@ def block_decode(x: torch.Tensor, norm1, eps1: float, wq, wk, wv, wo, norm2, eps
     fp8 = is_fp8(k_pool)
     if fp8:
         _scales(k_pool, k_scale, v_scale)
+    window, n_sink = int(window), int(n_sink)
     hidden, max_blocks = wup.shape[0], block_tables.shape[1]
     out = torch.empty_like(x)
     ws = _workspace(dev, _decode_workspace_bytes(m, num_q_heads, hkv, head_dim, bs, max_blocks, window,

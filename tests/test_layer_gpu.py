@@ -174,6 +174,25 @@ def test_decode_step_in_one_call_matches_modules(iva, dev, batch, kw):
         assert (a.double() - b.double()).norm() <= tol * b.double().norm()
 
 
+@pytest.mark.parametrize("window,sinks", [(48.0, 4), (48.9, 4), (0.0, 4), (None, 0)])
+def test_decode_step_window_types(iva, dev, window, sinks):
+    """A window read from a configuration as a float is truncated, as the attention ops do."""
+    M = iva.model
+    cfg = M.TransformerConfig(d_model=256, n_heads=4, n_layers=1, vocab_size=64, seq_len=128, dropout=0.0,
+                              attn_impl="hip_paged")
+    torch.manual_seed(3)
+    block = M.Transformer(cfg).to(dev, torch.bfloat16).eval().blocks[0]
+    prompt, x = (_randn((2, n, 256), n, dev, torch.bfloat16) for n in (80, 1))
+
+    def step(w):
+        cache = iva.PagedKVCache(2, 4, 64, 0, dev, torch.bfloat16, num_layers=1, max_seq_len=96)
+        kw = dict(sliding_window=w, sink_cfg={"sink_tokens": sinks})
+        with torch.no_grad():
+            return torch.stack([block(prompt, kv_cache=cache, **kw)[0][:, -1:], block(x, kv_cache=cache, **kw)[0]])
+
+    assert torch.equal(step(window), step(None if window is None else int(window)))
+
+
 @pytest.mark.parametrize("lengths,n", [([16, 16], 16), ([40, 40, 40], 1), ([33, 5, 100], 7), ([3], 5)])
 def test_chunk_slots_match_the_pool(iva, dev, lengths, n):
     """Slots found on the device equal the allocator's; positions without a page give -1."""
