@@ -253,17 +253,63 @@ def _linear_weight(m: nn.Module, x: torch.Tensor, n: Optional[int], k: int
     return w if cols == k and rows % 16 == 0 and k % 64 == 0 and n in (None, rows) else None
 
 
+# How many rows the few-row linear kernel takes, by the widths of what it computes.  Each
+# workgroup of the kernel reads all rows for its 16 columns and walks all of k, so it falls
+# behind the library's larger tiles and split walks with more rows and a longer k.  Against
+# that stands the host: a library product costs it 28 us, the kernel 13 (q, k and v in one
+# call 23 : 75, a feed-forward layer 26 : 87, a decode step's block 43 : 258).  So the lines lie
+# where the kernel's loss on the GPU outgrows what the calls save.  Figures: us per call,
+# kernel : library, on the GPU alone (calls queued) / as called one by one, bf16, weights from
+# HBM, the library's side with the norm and SwiGLU kernels.
+
+def _qkv_rows(k: int) -> int:
+    """Most rows of the products q, k and v in one launch."""
+    # 32 rows of k 2048 16.5 : 32.4 / 23 : 74; of 4096 40.7 : 32.8 / 42 : 75; 16 rows of 5120 32.7 : 29.7 /
+    # 34 : 75, of 8192 54 : 55 / 55 : 75; 32 of 8192 77 : 61 / 75 : 74.
+    return 32 if k <= 4096 else 16
+
+
+def _output_rows(k: int) -> int:
+    """Most rows of the attention's output projection, a single product."""
+    # 32 rows of k 2048 9.1 : 10.9 / 13 : 28; 16 of 4096 11.7 : 13.5 / 14 : 29 (fp16 12.1 : 10.5 / 14 : 28), 32
+    # 15.7 : 11.1 / 17 : 28; one of 5120 23.6 : 13.0 / 25 : 29, of 8192 28 : 25 / 29 : 29.
+    return 32 if k <= 2048 else 16 if k <= 4096 else 0
+
+
+def _ffn_rows(d: int, hidden: int) -> int:
+    """Most rows of gate, up, SwiGLU and down."""
+    # The down product, on its long k, loses first.  d 1024, 32 rows 24 : 38 / 27 : 89; 2048, 16 rows
+    # 42 : 43 / 42 : 88, 32 56 : 46 / 55 : 85; 3072, 4 rows 69 : 63 / 70 : 85, 32 104 : 65 / 101 : 89;
+    # 4096, 4 rows 98 : 96 / 98 : 99, 16 112 : 96 / 111 : 99; 8192, 4 rows 320 : 329 / 319 : 332, 16
+    # 380 : 346 / 375 : 350.
+    return 32 if d <= 2048 and hidden <= 8192 else 4
+
+
+def _block_rows(d: int, hidden: int) -> int:
+    """Most rows of a whole block."""
+    # d 2048, 32 rows 90 : 110 / 89 : 266; 3072, 16 rows 133 : 137 / 135 : 272, 32 169 : 132 / 169 : 283;
+    # 4096, 16 rows 166 : 182 / 168 : 280 (fp16 165 : 169), 32 210 : 181 / 209 : 284; 5120, 8 rows 288 : 381
+    # / 287 : 399, 32 404 : 316 / 403 : 335; 8192, 8 rows 440 : 455 / 438 : 471, 16 499 : 460 / 495 :
+    # 476.
+    return 32 if d <= 4096 and hidden <= 16384 else 8
+
+
+def _head_rows(k: int, n: int) -> int:
+    """Most rows of the vocabulary head, one product with many columns."""
+    # On the GPU: 32000 x 1024, 16 rows 17.1 : 17.4, 32 28.9 : 24.2; 16384 x 1024, 16 rows 11.4 : 10.0;
+    # 32000 x 512, one row 13.8 : 13.0, 16 16.5 : 13.1; 50304 x 768 23.2 : 18.4; 65536 x 1024, 16 rows
+    # 30.3 : 26.3; 32000 x 2048, one row 34.2 : 32.2, 16 36.4 : 32.6, x 4096 53.4 : 57.7, 16 75.4 : 58.5;
+    # 4096 x 2048, 16 rows 9.6 : 11.
+    return 16 if (k <= 1024 and n <= 32768) or (k <= 2048 and n <= 4096) else 0
+
+
+def _rows(x: torch.Tensor) -> int:
+    return x.numel() // x.shape[-1]
+
+
 def _few_rows(x: torch.Tensor) -> bool:
-    """Few enough rows for the linear kernel, which streams every weight once: at 16 rows it
-    takes 4.5 us where the library's three q / k / v products take 17, 4.0 against 5.6 us
-    (d_model 1024) and 10.3 against 14.4 us (hidden 4096) for the others, at 32 rows 5.9 / 5.4
-    / 14.1 us; past that the library's larger tiles win."""
+    """Rows the kernel takes at all."""
     return x.numel() <= LINEAR_MAX_ROWS * x.shape[-1]
-
-
-# The vocabulary head (32000 columns): 18.3 against 19.3 us at 16 rows, 29 against 19.5 us
-# at 32, where each workgroup's reads of the rows outweigh its weights.
-HEAD_MAX_ROWS = 16
 
 
 def _visible(q_pos: torch.Tensor, k_pos: torch.Tensor, window: Optional[int], n_sink: int
@@ -438,7 +484,8 @@ class PagedAttention(_AttentionBase):
 
     def _project(self, x):
         """q, k and v in one launch on a decode step's few rows."""
-        if _plain_mode() and _plain_input(x) and _few_rows(x) and not _has_any_global_hook():
+        if (_plain_mode() and _plain_input(x) and _rows(x) <= _qkv_rows(x.shape[-1])
+                and not _has_any_global_hook()):
             w = self._qkv_weights(x)
             if w is not None:
                 return self._split_heads(linear_rows(x, w))
@@ -471,7 +518,7 @@ class PagedAttention(_AttentionBase):
     def _output(self, out):
         if _plain_mode() and _plain_input(out) and _few_rows(out) and not _has_any_global_hook():
             w = _linear_weight(self._modules["o_proj"], out, None, out.shape[-1])
-            if w is not None:
+            if w is not None and _rows(out) <= _output_rows(w.shape[1]):
                 return linear_rows(out, (w,))
         return self.o_proj(out)
 
@@ -662,7 +709,7 @@ class FFN(nn.Module):
         if self.activation == "swiglu":
             if _plain_mode() and _plain_input(x) and _few_rows(x) and not _has_any_global_hook():
                 w = self._weights(x)
-                if w is not None:
+                if w is not None and _rows(x) <= _ffn_rows(x.shape[-1], w[0].shape[0]):
                     return linear_rows(linear_rows(x, w[:2], swiglu_pair=True), w[2:])
             up, gate = self.up_proj(x), self.gate_proj(x)
             if (_plain_mode() and _plain_input(up) and _plain_weight(gate, up)
@@ -738,7 +785,8 @@ class TransformerBlock(nn.Module):
             d = x.shape[-1]
             qkv, w = attn._qkv_weights(x), ffn._weights(x)
             wo = _linear_weight(attn._modules["o_proj"], x, d, attn.n_heads * attn.head_dim)
-            if qkv is not None and wo is not None and w is not None and w[2].shape[0] == d:
+            if (qkv is not None and wo is not None and w is not None and w[2].shape[0] == d
+                    and _rows(x) <= _block_rows(d, w[0].shape[0])):
                 if attn._decodes(x, attention_mask, kv_cache):
                     return self._decode_step(x, qkv, wo, w, kv_cache, sliding_window, sink_cfg)
                 in_norm = (x.numel() <= LINEAR_NORM_MAX_ROWS * x.shape[-1]
@@ -813,8 +861,9 @@ class Transformer(nn.Module):
 
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         w = self.token_embedding.weight if self.lm_head is None else self.lm_head.weight
-        if (_plain_mode() and _plain_input(x) and x.numel() <= HEAD_MAX_ROWS * x.shape[-1]
+        if (_plain_mode() and _plain_input(x) and _few_rows(x)
                 and _plain_weight(w, x) and w.dim() == 2 and w.shape[1] == x.shape[-1]
+                and _rows(x) <= _head_rows(w.shape[1], w.shape[0])
                 and w.shape[0] % 16 == 0 and w.shape[1] % 64 == 0):
             return linear_rows(x, (w,))
         return F.linear(x, w)
