@@ -144,12 +144,13 @@ __global__ __launch_bounds__(256) void append_vec_kernel(AppendArgs a) {
 // per wave (two: 15.0 against 12.0 us on the ragged chunks below).
 //
 // us against append_vec_kernel, 8 heads x 128 dims from HBM: 11 ragged chunks (4658 rows) 12.0 :
-// 16.7, 8 chunks of 4096 53.7 : 64.9, 16 of 512 15.1 : 14.7, starting mid-page 17.4 : 18.3, 300
+// 16.7, 8 chunks of 4096 53.7 : 64.9, 16 of 512 15.1 : 15.1, starting mid-page 17.5 : 19.0, 300
 // of 20 18.6 : 22.2; 32 heads, 16 chunks of 512 mid-page 52 : 84; 16 heads x 64, 16 of 512 14.3 :
 // 15.6.  Chosen from kRunTokens rows and kRunElems elements of K up: below, a window's one wave
 // per head is a long chain (512 rows of 8 heads 4.7 : 3.4, 2048 6.3 : 7.6; a decode step of 1024
 // scattered rows 13.2 : 11.0); head_dim 256 from four times that (300 x 20 rows 21.3 : 20.4, 16
-// chunks of 512 13.6 : 17.7).  Rows scattered singly gain nothing (8192 of them 67.9 : 66.7).
+// chunks of 512 13.6 : 17.7).  Rows scattered singly gain little (8192 of them 69.6 : 70.2, of
+// 32 heads 304 : 317; 2048 of 8 heads 19.0 : 20.7, of 32 heads 71.3 : 70.5).
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 constexpr int kRunTokens = 2048;
 constexpr int64_t kRunElems = 1 << 21;

@@ -57,9 +57,9 @@ __device__ inline float silu_mul(float u, float g) {
 // A wave normalizes one row of NC * 64 16-byte chunks (chunks past the row are masked):
 // out = round(round(x / sqrt(mean(x^2) + eps)) * w), with x = round(x + residual) first
 // when there is a residual, stored to `sum`.  The row stays in registers between the sum
-// of squares and the store, so it is read once.  8192 rows of 1024 (bf16): 7.8 us = 4.3 TB/s
-// against 65 us for nine torch operators, 11.3 us with the residual (+ 9 us as an operator);
-// 16 rows 2.1 us (launch and one round trip) against 21 us.
+// of squares and the store, so it is read once.  8192 rows of 1024 (bf16, from HBM): 8.2 us =
+// 4.1 TB/s against 66 us for nine torch operators, with the residual 13.5 us = 5.0 TB/s against
+// 74 us for ten; 16 rows 2.8 us (launch and one round trip) against 24 us.
 template <int DT, int NC>
 __global__ __launch_bounds__(256) void rms_norm_kernel(const void* x, const void* residual,
                                                        const void* weight, void* sum, void* out,
@@ -137,9 +137,10 @@ void launch_rms_norm(const void* x, const void* residual, const void* weight, vo
 // SwiGLU
 // ---------------------------------------------------------------------------
 
-// out = silu(up) * gate over n8 16-byte chunks: each thread takes two chunks a grid apart,
-// all four loads before the first store.  8192 x 4096 bf16: 32 us = 6.3 TB/s against 61 us
-// for silu and product as two torch operators.
+// out = silu(up) * gate over n8 16-byte chunks: each thread takes two chunks, 256 apart so that
+// a wave's accesses stay contiguous, all four loads before the first store.  8192 x 4096
+// bf16: 30 - 32 us = 6.3 - 6.6 TB/s against 61 - 64 us for silu and product as two torch
+// operators.
 template <int DT>
 __global__ __launch_bounds__(256) void swiglu_kernel(const Chunk16* up, const Chunk16* gate,
                                                      Chunk16* out, int64_t n8) {
@@ -462,8 +463,9 @@ constexpr int kLinearNormRows = 16;
 constexpr int kLinearNormMaxK = 2048;
 constexpr int kNormLdsRows = 4;
 
-// Workgroups of a launch: what the CUs hold at once (four of 4 waves, two of 8),
-// each taking tiles a grid apart.
+// Workgroups of a launch, each taking tiles a grid apart: four of 4 waves per CU, or two of 8.
+// The CUs hold that many at once in the plain and residual instances; the SwiGLU ones (two
+// matrices' loads in registers) run at half of it, and the rest follow as those end.
 constexpr int kLinearWaves = 256 * 16;
 
 template <int DT, int MT, int WAVES, int NORM, int EPI, bool ONE>

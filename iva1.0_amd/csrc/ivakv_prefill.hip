@@ -14,13 +14,13 @@
 // the pair's K and V tiles move HBM -> registers -> an LDS ring (eight buffers
 // for the pipelined loop, two otherwise) once per workgroup, and every wave
 // reads them from LDS in MFMA operand order (the pools' tile layout is kept in
-// LDS):
-//   S^T[key][row]  = K_page(16 x D) . Q^T(D x 16)        v_mfma 16x16x32, per page
+// LDS, page B's K rows swizzled):
+//   S^T[key][row]  = K(16 keys x D) . Q^T(D x 16)        v_mfma 16x16x32, two per pair
 //   O^T[dim][row] += V^T_pair(D x 32) . P^T(32 x 16)     v_mfma 16x16x32, per pair
-// The QK accumulator of lane l holds keys 4*(l/16)+r of row l%16 for each page
-// of the pair; those 8 values are exactly the k-slots of the PV MFMA's B
-// operand (slot 8*(l/16)+r = page A key 4*(l/16)+r, slot +4 = page B key), and
-// the V chunks of the two pages are paired the same way, so P never leaves
+// Each QK product takes half the keys of both pages, in the order that leaves lane l
+// with the scores of 8 consecutive keys of row l%16: keys 8*((l/16)&1) .. +7 of page
+// l/32 of the pair, four from each product.  Those are its k-slots of the PV MFMA's B
+// operand, and the same 8 keys of a V row are one contiguous LDS read, so P never leaves
 // registers.  Online softmax in fp32, log2 domain, as in the decode kernel.
 // A wave skips pairs that lie entirely after its last row; only the pairs on
 // its causal diagonal (or window edge, or the context's end) need masks.
@@ -64,7 +64,10 @@ struct PrefillArgs {
 // AGPRs) and one pair in flight.  The single launch at head_dim 64 (kSplit false) keeps one
 // pair in flight too and stays under 128 registers, so that two workgroups share a CU and
 // hide each other's barriers and loads: its walks are short (16 x 512 rows of 16 heads 37.1
-// -> 28.7 us, 16 chunks of <= 300 at <= 1000 keys 46.5 -> 39.6).  The split path's
+// -> 28.7 us, 16 chunks of <= 300 at <= 1000 keys 46.5 -> 39.6).  FP8 pages need 141
+// registers there (40 bytes of scratch under 128), so their workgroups stay one per CU; a
+// second pair in flight (177 registers) did not pay (16 x 512 rows of 16 heads 44.2 : 44.2
+// us, at 2048 keys of 32 / 8 heads 212 : 213, 16 x 128 rows 9.6 : 10.4).  The split path's
 // persistent workgroups are one per CU and keep the pipeline (93.4 against 95.5 us).
 template <int DT, int D, bool kSplit>
 struct PrefillShape {
@@ -448,7 +451,7 @@ __device__ __attribute__((always_inline)) inline void prefill_rows(
     read_k(buf, ka, kb);
     qk_mfma(ka, kb, sc);
   };
-  // This lane's 8 scores of row block rb (keys 4lq.. of page A, then of page B).
+  // This lane's 8 scores of row block rb: keys 8 (lq & 1) .. + 7 of page lq >> 1.
   auto lane_scores = [&](const PairS& sc, int rb, float (&sl)[8]) IVAKV_INLINE {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {

@@ -201,7 +201,8 @@ class LayeredKVCache:
 # tensors, outside autograd, autocast, tracing, functorch transforms and torch modes, and
 # (where a kernel spans several submodules) only over submodules that are exactly the
 # classes built here, without hooks or replaced forwards.  Anything else takes the torch
-# operators.
+# operators, torch.set_default_device and ``with torch.device(...)`` around the call among it:
+# both are torch function modes.
 
 def _plain_mode() -> bool:
     """No grad, autocast, trace, compile, functorch level, forward-mode level, torch
