@@ -101,28 +101,30 @@ def _require_gpu(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
-# The current stream's handle without a Stream object around it, where torch has it.
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+def _stream_handle(index: int) -> int:
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# The current stream's handle without a Stream object around it, and the current device
+# without torch's lazy initialisation, where torch has them.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _stream_handle)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def _stream(dev: torch.device) -> int:
-    if _raw_stream is not None and dev.index is not None:
-        return _raw_stream(dev.index)
-    return torch.cuda.current_stream(dev).cuda_stream
-
-
-_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+    return _raw_stream(dev.index) if dev.index is not None else torch.cuda.current_stream(dev).cuda_stream
 
 
 def _launch(dev: torch.device, name: str, *args) -> None:
     """Entry point ``name`` on ``dev``'s current stream, with ``dev`` current around the call:
     the library launches on the current device, and the default stream's handle is the same
     on every device."""
-    if dev.index == _current_device():
-        _abi.call(name, *args, _stream(dev))
+    index = dev.index
+    if index == _current_device():
+        _abi.call(name, *args, _raw_stream(index))
     else:
         with torch.cuda.device(dev):
-            _abi.call(name, *args, _stream(dev))
+            _abi.call(name, *args, _raw_stream(index))
 
 
 def _capturing(dev: torch.device) -> bool:
