@@ -12,7 +12,8 @@
  *     thread-local message describing it.
  *   - All pointers except `stream` and host scalars are DEVICE pointers owned by
  *     the caller (the library never allocates or frees device memory).
- *   - Work is enqueued asynchronously on `stream` (NULL = the default stream).
+ *   - Work is enqueued asynchronously on `stream` (NULL = the default stream) of the
+ *     current device, which has to be the one that holds the operands.
  *     Argument checks run on the host before any launch.
  *   - Integer indices read from device memory (slot ids, page ids, context
  *     lengths, positions) are bounds-checked inside the kernels: an out-of-range
