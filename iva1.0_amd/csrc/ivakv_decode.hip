@@ -50,12 +50,18 @@ constexpr int partial_wgs_per_cu(int D) { return D == 256 ? 1 : 2; }
 constexpr int kStreamWaves = 4;
 constexpr int kStreamThreads = 64 * kStreamWaves;
 constexpr int kMaxStreamWaves = 4096;
-// Fewest tiles worth giving a wave: two (a ring's worth) while that makes at most kFewWaves
-// waves (8 units of 64 pages 12.9 -> 11.2 us, 64 units of <= 48 pages 14.7 -> 13.6 us against
-// four each), four from there (64 units of <= 96 pages 15.6 us, 16.4 at two or three).
-constexpr int kMinTilesPerWave = 2;
-constexpr int kTilesPerWave = 4;
-constexpr int kFewWaves = 800;
+// Tiles a wave is given at least: four, or two (a ring's worth) while that makes at most
+// kTwoTilesMax / 2 waves and leaves a unit few enough partials to merge.  us at four : two, D 128
+// fp16: 8 units of 64 pages 12.9 : 11.2, 64 units of <= 48 pages 14.7 : 13.6; one unit of 130 tiles
+// 12.3 : 11.9, of 400 11.2 : 12.2, of 1000 13.1 : 16.1; 12 units of 160 11.0 : 12.3 (1920 tiles).  The
+// longer a tile takes, the more tiles per unit pay: fp32 and D 256, 200 tiles per unit 0.95
+// of the time, 300 0.97, 500 1.02; fp32 at D 256 0.86 at 1000.
+constexpr int kTwoTilesMax = 1600;
+int64_t two_tiles_max(int64_t units, int head_dim, int esize) {
+  if (head_dim == 256 && esize == 4) return kTwoTilesMax;
+  const int64_t most = units * (head_dim == 256 || esize == 4 ? 256 : 128);
+  return most < kTwoTilesMax ? most : kTwoTilesMax;
+}
 constexpr int kMaxStreamBatch = 8192;
 // Stream walk workgroups per CU from the bytes one ring slot holds (K + V of one
 // tile).  One 4-wave workgroup per CU keeps 2 x 8 KiB slots per wave in flight at
@@ -80,6 +86,7 @@ struct DecodeArgs {
   float scale_log2;
   int window, n_sink, part_pages, n_parts_max;
   int n_waves;         // stream: waves launched
+  int two_tiles_max;   // stream: tiles of the batch up to which a wave takes two
   // Fused append (ivakv_decode_append_attn): position L-1 of every sequence is the new
   // token, whose rows come from k_new / v_new ([B][Hkv][D] dense) instead of the pool.
   const void* k_new;
@@ -789,13 +796,9 @@ __device__ inline int64_t div_nn(int64_t n, int64_t d) {
   return n / d;
 }
 
-// Waves that share T tiles: kMinTilesPerWave each, which is one round trip of the ring, up to
-// kFewWaves waves; beyond that many the partials' merge costs more than the shorter walks
-// save, until every wave has kTilesPerWave.
-__device__ inline int64_t stream_waves(int64_t T, int n_waves) {
-  const int64_t few = (T + kMinTilesPerWave - 1) / kMinTilesPerWave;
-  const int64_t many = (T + kTilesPerWave - 1) / kTilesPerWave;
-  const int64_t want = few <= kFewWaves ? few : many > kFewWaves ? many : kFewWaves;
+// Waves that share T tiles: two or four each.
+__device__ inline int64_t stream_waves(int64_t T, int n_waves, int two_max) {
+  const int64_t want = T <= two_max ? (T + 1) >> 1 : (T + 3) >> 2;
   return want < n_waves ? (want > 0 ? want : 1) : n_waves;
 }
 
@@ -804,7 +807,7 @@ __device__ inline int64_t stream_waves(int64_t T, int n_waves) {
 // start(k + 1)).
 struct WaveSplit {
   int64_t T, W;
-  __device__ WaveSplit(int64_t T_, const DecodeArgs& a) : T(T_), W(stream_waves(T_, a.n_waves)) {}
+  __device__ WaveSplit(int64_t T_, const DecodeArgs& a) : T(T_), W(stream_waves(T_, a.n_waves, a.two_tiles_max)) {}
   __device__ int64_t start(int64_t k) const { return div_nn(k * T, W); }
   __device__ int64_t owner(int64_t t) const { return div_nn((t + 1) * W - 1, T); }
 };
@@ -1452,7 +1455,7 @@ int decode_entry(Stage stage, const char* name, const void* q, const void* k_poo
   a.n_sink = n_sink;
   a.part_pages = plan.part_pages;
   a.n_parts_max = plan.n_parts_max;
-  a.n_waves = 0;
+  a.n_waves = a.two_tiles_max = 0;
   a.k_new = k_new;
   a.v_new = v_new;
   a.fused = stage == kFused;
@@ -1463,6 +1466,7 @@ int decode_entry(Stage stage, const char* name, const void* q, const void* k_poo
     const int esize = fp8 ? 1 : dtype_size(dtype);
     const int wgs = stream_workgroups(walk_wgs_per_cu(2 * (int64_t)head_dim * kBS * esize));
     a.n_waves = wgs * kStreamWaves;
+    a.two_tiles_max = (int)two_tiles_max((int64_t)batch * num_kv_heads, head_dim, esize);
     const size_t smem = sizeof(int32_t) * ((size_t)batch + 1 + kStreamThreads);
     const dim3 grid((unsigned)wgs);
     if (fp8) {
