@@ -53,13 +53,17 @@ constexpr int kMaxStreamWaves = 4096;
 // Tiles a wave is given at least: four, or two (a ring's worth) while that makes at most
 // kTwoTilesMax / 2 waves and leaves a unit few enough partials to merge.  us at four : two, D 128
 // fp16: 8 units of 64 pages 12.9 : 11.2, 64 units of <= 48 pages 14.7 : 13.6; one unit of 130 tiles
-// 12.3 : 11.9, of 400 11.2 : 12.2, of 1000 13.1 : 16.1; 12 units of 160 11.0 : 12.3 (1920 tiles).  The
-// longer a tile takes, the more tiles per unit pay: fp32 and D 256, 200 tiles per unit 0.95
-// of the time, 300 0.97, 500 1.02; fp32 at D 256 0.86 at 1000.
+// 12.3 : 11.9, of 400 11.2 : 12.2, of 1000 13.1 : 16.1; 12 units of 160 11.0 : 12.3 (1920 tiles).  By
+// tiles per unit, time at two over time at four: 16-bit pages to D 128 100 0.93, 160 0.98, 200
+// 1.00, 300 1.03; where a tile takes longer (fp32, D 256) 200 0.95, 300 0.97, 500 1.01; fp32 at
+// D 256 0.86 at 1000.  Past kTwoTilesMax, units of at most kLevelTiles on average keep the waves
+// at that number until four tiles each make as many (1601 .. 1700 tiles in units of <= 60 0.90
+// of the time, .. 2500 0.98; in units of 130 .. 200 1.11).
 constexpr int kTwoTilesMax = 1600;
+constexpr int kLevelTiles = 60;
 int64_t two_tiles_max(int64_t units, int head_dim, int esize) {
   if (head_dim == 256 && esize == 4) return kTwoTilesMax;
-  const int64_t most = units * (head_dim == 256 || esize == 4 ? 256 : 128);
+  const int64_t most = units * (head_dim == 256 || esize == 4 ? 384 : 192);
   return most < kTwoTilesMax ? most : kTwoTilesMax;
 }
 constexpr int kMaxStreamBatch = 8192;
@@ -87,6 +91,7 @@ struct DecodeArgs {
   int window, n_sink, part_pages, n_parts_max;
   int n_waves;         // stream: waves launched
   int two_tiles_max;   // stream: tiles of the batch up to which a wave takes two
+  int64_t level_max;   // and up to which the waves are not fewer than for kTwoTilesMax
   // Fused append (ivakv_decode_append_attn): position L-1 of every sequence is the new
   // token, whose rows come from k_new / v_new ([B][Hkv][D] dense) instead of the pool.
   const void* k_new;
@@ -796,9 +801,11 @@ __device__ inline int64_t div_nn(int64_t n, int64_t d) {
   return n / d;
 }
 
-// Waves that share T tiles: two or four each.
-__device__ inline int64_t stream_waves(int64_t T, int n_waves, int two_max) {
-  const int64_t want = T <= two_max ? (T + 1) >> 1 : (T + 3) >> 2;
+// Waves that share T tiles: two or four each, or those of kTwoTilesMax tiles.
+__device__ inline int64_t stream_waves(int64_t T, const DecodeArgs& a) {
+  const int n_waves = a.n_waves;
+  int64_t want = T <= a.two_tiles_max ? (T + 1) >> 1 : (T + 3) >> 2;
+  if (T > kTwoTilesMax && T <= a.level_max && want < kTwoTilesMax / 2) want = kTwoTilesMax / 2;
   return want < n_waves ? (want > 0 ? want : 1) : n_waves;
 }
 
@@ -807,7 +814,7 @@ __device__ inline int64_t stream_waves(int64_t T, int n_waves, int two_max) {
 // start(k + 1)).
 struct WaveSplit {
   int64_t T, W;
-  __device__ WaveSplit(int64_t T_, const DecodeArgs& a) : T(T_), W(stream_waves(T_, a.n_waves, a.two_tiles_max)) {}
+  __device__ WaveSplit(int64_t T_, const DecodeArgs& a) : T(T_), W(stream_waves(T_, a)) {}
   __device__ int64_t start(int64_t k) const { return div_nn(k * T, W); }
   __device__ int64_t owner(int64_t t) const { return div_nn((t + 1) * W - 1, T); }
 };
@@ -1348,7 +1355,8 @@ int stream_workgroups(int per_cu) {
 //   Fewer units than CUs: one CU reads about 50 GB/s, so the walk by one workgroup stays ahead
 //   of the stream walk's fixed 11 us only up to kSingleUnitBytes of K and V (32 tiles of 8 KiB:
 //   10.2 - 11.0 against 11.0 - 13.3 us; 48: 12.8 - 13.6 against 11.2 - 13.6), and smaller tiles do
-//   not come faster (FP8, 48 tiles of 4 KiB: 11.9 against 11.5).
+//   not come faster (FP8, 48 tiles of 4 KiB: 11.9 against 11.5; at D 256 its 32 tiles of 8 KiB
+//   13.6 against 12.4, but 12.0 against 18.3 where they are 12 long on average).
 constexpr int kSinglePartitionMaxPages = 64;
 constexpr int kSingleFewMaxPages = 32;
 constexpr int64_t kSingleUnitBytes = 256 * 1024;
@@ -1456,6 +1464,7 @@ int decode_entry(Stage stage, const char* name, const void* q, const void* k_poo
   a.part_pages = plan.part_pages;
   a.n_parts_max = plan.n_parts_max;
   a.n_waves = a.two_tiles_max = 0;
+  a.level_max = 0;
   a.k_new = k_new;
   a.v_new = v_new;
   a.fused = stage == kFused;
@@ -1466,7 +1475,9 @@ int decode_entry(Stage stage, const char* name, const void* q, const void* k_poo
     const int esize = fp8 ? 1 : dtype_size(dtype);
     const int wgs = stream_workgroups(walk_wgs_per_cu(2 * (int64_t)head_dim * kBS * esize));
     a.n_waves = wgs * kStreamWaves;
-    a.two_tiles_max = (int)two_tiles_max((int64_t)batch * num_kv_heads, head_dim, esize);
+    const int64_t units = (int64_t)batch * num_kv_heads;
+    a.two_tiles_max = (int)two_tiles_max(units, head_dim, esize);
+    a.level_max = kLevelTiles * units;
     const size_t smem = sizeof(int32_t) * ((size_t)batch + 1 + kStreamThreads);
     const dim3 grid((unsigned)wgs);
     if (fp8) {
