@@ -126,10 +126,11 @@ int ivakv_decode_workspace_size(int batch, int num_q_heads, int num_kv_heads,
  * workgroup each) merged the same way.  With partition_pages <= 0, a batch of at
  * least one (sequence, kv head) unit per CU on tables of at most 64 effective
  * pages, or of fewer units on tables of at most 32 pages and 256 KiB of K and V a
- * unit, takes one partition per sequence in a single launch with no merge (with
- * one to four units per CU the call then accepts a null workspace;
- * ivakv_decode_workspace_size reports the stream walk's need in every case, which
- * covers it).
+ * unit, takes one partition per sequence in a single launch with no merge; from four
+ * units per CU on, only to head_dim 128 and where the pages per unit repay the
+ * workgroups.  With one to four units per CU the single launch accepts a null
+ * workspace; ivakv_decode_workspace_size reports the stream walk's need in every
+ * case, which covers it.
  * Supported: block_size 16, head_dim 64/128/256, num_q_heads/num_kv_heads
  * (the GQA group) any integer from 1 to 16.
  * Replaces: the cache branch of AttentionTorch.forward -- scores, causal /
@@ -176,10 +177,9 @@ int ivakv_decode_attn_merge(const void* q, const void* k_pool, const void* v_poo
  * attended together with positions < L-1 read from the pools.  Same result as
  * ivakv_append of those rows followed by ivakv_decode_attn, in two launches
  * instead of three: the pool walk skips position L-1 and the merge scores the new
- * token straight from k_new.  When the batch has one to four (sequence, kv head)
- * units per CU of the device and the table holds at most 64 effective pages per
- * sequence (max_blocks, or the window and sinks), one launch: a workgroup per unit
- * walks it, merges its waves in LDS, folds in the new token and stores its rows.
+ * token straight from k_new.  On short tables (as ivakv_decode_attn takes a single
+ * launch), one launch: a workgroup per unit walks it, merges its waves in LDS, folds
+ * in the new token and stores its rows.
  * Workspace: ivakv_decode_workspace_size with partition_pages <= 0 (enough for
  * either).  Supported geometry as ivakv_decode_attn, batch <= 8192.
  * Replaces: the append + score sequence of AttentionTorch.forward with a cache

@@ -1345,11 +1345,11 @@ int stream_workgroups(int per_cu) {
 // Calls on short tables take one partition per sequence: a workgroup per (sequence, kv head)
 // unit walks it, merges its waves in LDS, folds the new token and writes out, with no merge
 // kernel.  Returns the partition size for that, or 0 for the stream walk.
-//   From one unit per CU: tables up to 64 pages.  us, single launch against walk + merge, 8 kv
-//   heads, D 128, all at the table's width / lengths spread from 1 to it: 256 units of 32
-//   pages 15.7 : 19.8 / 13.1 : 18.6, of 64 26.0 : 29.8 / 19.7 : 23.6; 512 of 64 45.3 : 50.7 / 31.4 :
-//   38.3; 1024 of 32 49.3 : 52.7 / 33.0 : 41.7; 2048 of 16 57.3 : 59.3 / 38.3 : 47.6; FP8 1024 of 64
-//   52.3 : 59.0 / 40.7 : 46.0.  Wider tables tell too little of the lengths: at 96 pages the two
+//   From one unit per CU: tables up to 64 pages, from four on where single_pays().  us, single
+//   launch against walk + merge, 8 kv heads, D 128, all at the table's width / lengths spread
+//   from 1 to it: 256 units of 32 pages 15.7 : 19.8 / 13.1 : 18.6, of 64 26.0 : 29.8 / 19.7 :
+//   23.6; 512 of 64 45.3 : 50.7 / 31.4 : 38.3; 1024 of 32 49.3 : 52.7 / 33.0 : 41.7; 2048 of 16
+//   57.3 : 59.3 / 38.3 : 47.6; FP8 1024 of 64 52.3 : 59.0 / 40.7 : 46.0.  Wider tables tell too little of the lengths: at 96 pages the two
 //   meet (256 units spread to 96: 25.9 : 27.9), past them one long unit's walk by one workgroup
 //   would set the time.
 //   Fewer units than CUs: one CU reads about 50 GB/s, so the walk by one workgroup stays ahead
@@ -1367,15 +1367,42 @@ int device_cus() {
     return 0;
   return cus;
 }
+
+// Four or more units per CU.  A workgroup has a fixed cost (start, the query rows, the merge of
+// its waves) that the stream walk has once per wave of the chip, and two share a CU (one at
+// D 256).  It is repaid at `even` pages per unit, at fewer while the rounds of workgroups cost
+// less than the walk's own start and its merge launch:
+//   (units / (2 CUs)) * (even - pages) < rounds.
+// us, single launch against walk + merge, units of all one length:
+//   fp16 D 128, fused   2048 x 2 pages 22 : 22, 4096 x 2 38 : 34, x 4 45 : 46, 8192 x 4 81 : 80, x 6
+//                       102 : 104, 16384 x 2 123 : 101, x 4 156 : 152
+//   attention alone     2048 x 3 18 : 16, 4096 x 2 27 : 21, x 6 36 : 38, 16384 x 2 100 : 68
+//   fp16 D 64, fused    4096 x 2 22 : 24, 8192 x 2 38 : 35, 16384 x 2 69 : 61, x 4 83 : 92
+//   FP8 D 128, fused    2048 x 4 25 : 24, 4096 x 8 48 : 54, x 4 44 : 39, 8192 x 8 87 : 92, x 4 82 : 64
+//   FP8 D 64, fused     4096 x 4 28 : 26, x 6 29 : 30, 16384 x 4 94 : 74, x 8 98 : 100
+//   fp32 D 128, fused   1536 x 2 34 : 31, 2048 x 8 65 : 67, x 4 51 : 45, 4096 x 4 90 : 79
+//   D 256: never (1024 x 3 pages 36 : 29, FP8 39 : 24 at four, fp32 67 : 50; 4096 x 2 108 : 59)
+bool single_pays(int64_t units, int64_t cus, int pages, int head_dim, int esize, bool fused) {
+  if (head_dim == 256) return false;
+  const int tile = 2 * kBS * head_dim * esize;
+  const int alone = fused ? 0 : 1;
+  const int even = esize == 1 ? (head_dim == 64 ? 9 : 12 + alone)
+                   : tile <= 4096 ? 5 + alone : tile <= 8192 ? 7 + alone : 13;
+  const int rounds = esize == 1 ? 35 : fused ? 25 : 21;
+  return units * (even - pages) < 2 * cus * rounds;
+}
+
 int single_partition_pages(int batch, int num_kv_heads, int head_dim, int esize, int max_blocks,
-                           int window, int n_sink) {
+                           int window, int n_sink, bool fused) {
   const int max_eff = max_effective_pages(max_blocks, window, n_sink, kBS);
-  const int cus = device_cus();
+  const int64_t cus = device_cus(), units = (int64_t)batch * num_kv_heads;
   if (max_eff <= 0 || batch > kMaxStreamBatch || cus <= 0) return 0;
   int64_t limit = kSinglePartitionMaxPages;
-  if ((int64_t)batch * num_kv_heads < cus) {
+  if (units < cus) {
     limit = kSingleUnitBytes / (2 * (int64_t)kBS * head_dim * esize);
     if (limit > kSingleFewMaxPages) limit = kSingleFewMaxPages;
+  } else if (units >= 4 * cus && !single_pays(units, cus, max_eff, head_dim, esize, fused)) {
+    return 0;
   }
   return max_eff <= limit ? max_eff : 0;
 }
@@ -1389,7 +1416,8 @@ int make_decode_plan(const char* name, Stage stage, int batch, int num_q_heads, 
   int st = make_plan(name, stage, batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks,
                      window, n_sink, 0, plan);
   const int pp = block_size == kBS && n_sink >= 0 && num_kv_heads > 0 && head_dim > 0
-                     ? single_partition_pages(batch, num_kv_heads, head_dim, esize, max_blocks, window, n_sink)
+                     ? single_partition_pages(batch, num_kv_heads, head_dim, esize, max_blocks, window, n_sink,
+                                              stage == kFused)
                      : 0;
   if (pp <= 0) return st;
   const size_t stream_bytes = plan->ws_bytes;
