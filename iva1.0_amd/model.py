@@ -206,9 +206,9 @@ class LayeredKVCache:
 
 def _plain_mode() -> bool:
     """No grad, autocast, trace, compile, functorch level, forward-mode level, torch
-    function or dispatch mode is active.  Asked before anything of a tensor is looked at:
-    under a functorch transform a tensor has no address to look at.  Compilation is asked
-    first of all: the compiler takes that as a constant and follows nothing of the rest."""
+    function or dispatch mode is active.  Asked before a tensor's address and layout: under a
+    functorch transform it has none.  Compilation is asked first of all: the compiler takes
+    that as a constant and follows nothing of the rest."""
     return not (torch.compiler.is_compiling() or torch.is_grad_enabled()
                 or torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack()
                 or torch.is_autocast_enabled("cuda")
@@ -217,10 +217,19 @@ def _plain_mode() -> bool:
                 or fwAD._current_level >= 0)
 
 
-def _plain_input(x: Any) -> bool:
+def _plain_type(x: Any) -> bool:
     return (type(x) is torch.Tensor and x.is_cuda
-            and (x.dtype is torch.bfloat16 or x.dtype is torch.float16) and x.is_contiguous()
-            and x.numel() > 0 and not x.is_neg() and not x.data_ptr() & 15)
+            and (x.dtype is torch.bfloat16 or x.dtype is torch.float16))
+
+
+def _plain_layout(x: torch.Tensor) -> bool:
+    return x.is_contiguous() and x.numel() > 0 and not x.is_neg() and not x.data_ptr() & 15
+
+
+def _plain(x: Any) -> bool:
+    """A tensor and a moment the layer kernels stand in for: its type, then the mode, then
+    what only a tensor outside every transform can be asked."""
+    return _plain_type(x) and _plain_mode() and _plain_layout(x)
 
 
 def _plain_weight(w: Any, x: torch.Tensor) -> bool:
@@ -280,10 +289,13 @@ def _output_rows(k: int) -> int:
 def _ffn_rows(d: int, hidden: int) -> int:
     """Most rows of gate, up, SwiGLU and down."""
     # The down product, on its long k, loses first.  d 1024, 32 rows 24 : 38 / 27 : 89; 2048, 16 rows
-    # 42 : 43 / 42 : 88, 32 56 : 46 / 55 : 85; 3072, 4 rows 69 : 63 / 70 : 85, 32 104 : 65 / 101 : 89;
-    # 4096, 4 rows 98 : 96 / 98 : 99, 16 112 : 96 / 111 : 99; 8192, 4 rows 320 : 329 / 319 : 332, 16
-    # 380 : 346 / 375 : 350.
-    return 32 if d <= 2048 and hidden <= 8192 else 4
+    # 42 : 43 / 42 : 88, 32 56 : 46 / 55 : 85; 3072, 16 rows 80 : 66 / 80 : 86, 32 104 : 65 / 101 : 89;
+    # 4096, 4 rows 98 : 96 / 98 : 99, 16 112 : 96 / 111 : 99 (in a block of modules, which the host
+    # bounds to that width, 7 rows 367 : 425 as called), 32 142 : 101; 8192, 4 rows 320 : 329 / 319 :
+    # 332, 16 380 : 346 / 375 : 350.
+    if d <= 2048 and hidden <= 8192:
+        return 32
+    return 16 if d <= 4096 and hidden <= 16384 else 4
 
 
 def _block_rows(d: int, hidden: int) -> int:
@@ -300,8 +312,8 @@ def _head_rows(k: int, n: int) -> int:
     # On the GPU: 32000 x 1024, 16 rows 17.1 : 17.4, 32 28.9 : 24.2; 16384 x 1024, 16 rows 11.4 : 10.0;
     # 32000 x 512, one row 13.8 : 13.0, 16 16.5 : 13.1; 50304 x 768 23.2 : 18.4; 65536 x 1024, 16 rows
     # 30.3 : 26.3; 32000 x 2048, one row 34.2 : 32.2, 16 36.4 : 32.6, x 4096 53.4 : 57.7, 16 75.4 : 58.5;
-    # 4096 x 2048, 16 rows 9.6 : 11.
-    return 16 if (k <= 1024 and n <= 32768) or (k <= 2048 and n <= 4096) else 0
+    # 512 x 4096, one row 8.3 : 14.6, 16 11.1 : 14.6.
+    return 16 if (k <= 1024 and n <= 32768) or (k <= 4096 and n <= 4096) else 0
 
 
 def _rows(x: torch.Tensor) -> int:
@@ -485,7 +497,7 @@ class PagedAttention(_AttentionBase):
 
     def _project(self, x):
         """q, k and v in one launch on a decode step's few rows."""
-        if (_plain_mode() and _plain_input(x) and _rows(x) <= _qkv_rows(x.shape[-1])
+        if (_plain(x) and _rows(x) <= _qkv_rows(x.shape[-1])
                 and not _has_any_global_hook()):
             w = self._qkv_weights(x)
             if w is not None:
@@ -517,7 +529,7 @@ class PagedAttention(_AttentionBase):
                 v.view(b, s, self.n_kv_heads, self.head_dim))
 
     def _output(self, out):
-        if _plain_mode() and _plain_input(out) and _few_rows(out) and not _has_any_global_hook():
+        if _plain(out) and _few_rows(out) and not _has_any_global_hook():
             w = _linear_weight(self._modules["o_proj"], out, None, out.shape[-1])
             if w is not None and _rows(out) <= _output_rows(w.shape[1]):
                 return linear_rows(out, (w,))
@@ -674,7 +686,7 @@ class RMSNorm(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not torch.jit.is_scripting():  # (what is inside is not scripted)
-            if _plain_mode() and _plain_input(x) and self._kernel_takes(x):
+            if _plain(x) and self._kernel_takes(x):
                 return rms_norm(x, self.weight, self.eps)
         xf = x.float()
         y = xf / torch.sqrt(torch.mean(xf * xf, dim=-1, keepdim=True) + self.eps)
@@ -708,12 +720,12 @@ class FFN(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.activation == "swiglu":
-            if _plain_mode() and _plain_input(x) and _few_rows(x) and not _has_any_global_hook():
+            if _plain(x) and _few_rows(x) and not _has_any_global_hook():
                 w = self._weights(x)
                 if w is not None and _rows(x) <= _ffn_rows(x.shape[-1], w[0].shape[0]):
                     return linear_rows(linear_rows(x, w[:2], swiglu_pair=True), w[2:])
             up, gate = self.up_proj(x), self.gate_proj(x)
-            if (_plain_mode() and _plain_input(up) and _plain_weight(gate, up)
+            if (_plain(up) and _plain_weight(gate, up)
                     and gate.shape == up.shape and up.numel() % 8 == 0):
                 hidden = swiglu(up, gate)
             else:
@@ -740,7 +752,7 @@ class TransformerBlock(nn.Module):
 
     def forward(self, x, attention_mask=None, kv_cache=None, rope_state=None, sliding_window=None,
                 sink_cfg=None, router_temp=None, hrm_state=None):
-        if _plain_mode() and _plain_input(x) and self._fusable(x):
+        if _plain(x) and self._fusable(x):
             return (*self._forward_fused(x, attention_mask, kv_cache, sliding_window, sink_cfg), {})
         attn_out, new_kv_cache = self.attention(self.norm1(x), attention_mask=attention_mask,
                                                 kv_cache=kv_cache, rope_state=rope_state,
@@ -801,7 +813,7 @@ class TransformerBlock(nn.Module):
                 out, cache = attn._attend_rows(
                     x, lambda y: attn._split_heads(normed(y, n1, qkv)), attention_mask, kv_cache,
                     sliding_window, sink_cfg)
-                if _plain_input(out):
+                if _plain_type(out) and _plain_layout(out):
                     x = linear_rows(out, (wo,), residual=x)
                 else:
                     x = x + attn.o_proj(out)
@@ -862,7 +874,7 @@ class Transformer(nn.Module):
 
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         w = self.token_embedding.weight if self.lm_head is None else self.lm_head.weight
-        if (_plain_mode() and _plain_input(x) and _few_rows(x)
+        if (_plain(x) and _few_rows(x)
                 and _plain_weight(w, x) and w.dim() == 2 and w.shape[1] == x.shape[-1]
                 and _rows(x) <= _head_rows(w.shape[1], w.shape[0])
                 and w.shape[0] % 16 == 0 and w.shape[1] % 64 == 0):

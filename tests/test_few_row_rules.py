@@ -22,8 +22,8 @@ def taken(iva, monkeypatch):
         return x if residual is None else (x, x)
 
     for name, value in dict(linear_rows=linear_rows, rms_norm=rms_norm, swiglu=lambda u, g: u,
-                            _plain_mode=lambda: True, _plain_input=lambda x: True,
-                            _plain_weight=lambda w, x: True).items():
+                            _plain=lambda x: True, _plain_type=lambda x: True,
+                            _plain_layout=lambda x: True, _plain_weight=lambda w, x: True).items():
         monkeypatch.setattr(M, name, value)
     # the attention itself: its projections' rows come out as they went in
     monkeypatch.setattr(M.PagedAttention, "_attend_rows",
@@ -59,7 +59,8 @@ def test_wide_block_leaves_it(iva, taken, d, rows):
 
 @pytest.mark.parametrize("d,mult,rows,kernel", [
     (256, 4, 32, True), (1024, 8, 32, True), (2048, 4, 32, True), (3072, 4, 4, True), (8192, 4, 4, True),
-    (2048, 8, 16, False), (3072, 4, 5, False), (4096, 4, 16, False), (8192, 4, 16, False), (1024, 4, 33, False)])
+    (3072, 4, 16, True), (4096, 4, 16, True), (2048, 8, 17, False), (3072, 4, 17, False), (4096, 4, 32, False),
+    (8192, 4, 16, False), (1024, 4, 33, False)])
 def test_ffn(iva, taken, d, mult, rows, kernel):
     _block(iva, d, mult).ffn(_x(rows, d))
     assert bool(taken) == kernel
@@ -74,9 +75,9 @@ def test_attention_alone(iva, taken, d, rows, qkv, o):
 
 
 @pytest.mark.parametrize("d,vocab,rows,kernel", [
-    (1024, 32000, 16, True), (256, 32000, 1, True), (2048, 4096, 16, True), (512, 512, 17, False),
+    (1024, 32000, 16, True), (256, 32000, 1, True), (2048, 4096, 16, True), (4096, 512, 16, True), (512, 512, 17, False),
     (768, 50304, 1, False), (1024, 65536, 4, False), (1536, 32000, 1, False), (2048, 32000, 1, False),
-    (4096, 32000, 8, False), (4096, 512, 1, False), (8192, 128256, 16, False)])
+    (4096, 32000, 8, False), (8192, 512, 1, False), (8192, 128256, 16, False)])
 def test_head(iva, taken, d, vocab, rows, kernel):
     head = iva.Transformer.__new__(iva.Transformer)
     torch.nn.Module.__init__(head)
