@@ -268,14 +268,30 @@ def last_error() -> str:
     return msg.decode() if msg else ""
 
 
+class ForeignStream(int):
+    """The handle of a stream of a device that is not the current one: ``enter()`` gives the
+    context in which it is."""
+
+    @classmethod
+    def of(cls, handle: int, enter) -> "ForeignStream":
+        stream = cls(handle)
+        stream.enter = enter
+        return stream
+
+
 _FUNCS: dict = {}
 
 
 def call(name: str, *args) -> None:
-    """Calls entry point ``name``; raises IvakvError on a non-zero status."""
+    """Calls entry point ``name``, whose last argument is the stream if it launches; raises
+    IvakvError on a non-zero status."""
     fn = _FUNCS.get(name)
     if fn is None:
         fn = _FUNCS[name] = getattr(lib(), name)
-    status = fn(*args)
+    if type(args[-1]) is ForeignStream:
+        with args[-1].enter():
+            status = fn(*args)
+    else:
+        status = fn(*args)
     if status != OK:
         raise IvakvError(name, status, last_error())

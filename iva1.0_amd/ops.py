@@ -15,7 +15,7 @@ from __future__ import annotations
 
 import ctypes
 import math
-from functools import lru_cache
+from functools import lru_cache, partial
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -112,19 +112,13 @@ _current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device
 
 
 def _stream(dev: torch.device) -> int:
-    return _raw_stream(dev.index) if dev.index is not None else torch.cuda.current_stream(dev).cuda_stream
-
-
-def _launch(dev: torch.device, name: str, *args) -> None:
-    """Entry point ``name`` on ``dev``'s current stream, with ``dev`` current around the call:
-    the library launches on the current device, and the default stream's handle is the same
-    on every device."""
-    index = dev.index
-    if index == _current_device():
-        _abi.call(name, *args, _raw_stream(index))
-    else:
-        with torch.cuda.device(dev):
-            _abi.call(name, *args, _raw_stream(index))
+    """The handle of ``dev``'s current stream.  The library launches on the current device, and
+    the default stream's handle is the same on every device: where ``dev`` is not current,
+    the handle carries the context that makes it so for the call."""
+    index, current = dev.index, _current_device()
+    if index == current or index is None:
+        return _raw_stream(current)
+    return _abi.ForeignStream.of(_raw_stream(index), partial(torch.cuda.device, dev))
 
 
 def _capturing(dev: torch.device) -> bool:
@@ -194,16 +188,16 @@ def kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_pool: torch.Tensor, v_
         pos = _i32_row(rope_positions, "rope_positions")
         if pos.numel() != n_tok or pos.device != dev:
             raise ValueError(f"rope_positions must be {n_tok} int32 values on {dev}")
-        _launch(dev, "ivakv_append_rope", k_new.data_ptr(), v_new.data_ptr(),
-                k_new.stride(0), k_new.stride(1), v_new.stride(0), v_new.stride(1),
-                k_pool.data_ptr(), v_pool.data_ptr(), slot_mapping.data_ptr(), pos.data_ptr(),
-                n_tok, hkv, head_dim, bs, num_pages, float(rope_theta),
-                dtype_code(k_pool.dtype))
+        _abi.call("ivakv_append_rope", k_new.data_ptr(), v_new.data_ptr(),
+                  k_new.stride(0), k_new.stride(1), v_new.stride(0), v_new.stride(1),
+                  k_pool.data_ptr(), v_pool.data_ptr(), slot_mapping.data_ptr(), pos.data_ptr(),
+                  n_tok, hkv, head_dim, bs, num_pages, float(rope_theta),
+                  dtype_code(k_pool.dtype), _stream(dev))
         return
-    _launch(dev, "ivakv_append", k_new.data_ptr(), v_new.data_ptr(),
-            k_new.stride(0), k_new.stride(1), v_new.stride(0), v_new.stride(1),
-            k_pool.data_ptr(), v_pool.data_ptr(), slot_mapping.data_ptr(),
-            n_tok, hkv, head_dim, bs, num_pages, dtype_code(k_pool.dtype))
+    _abi.call("ivakv_append", k_new.data_ptr(), v_new.data_ptr(),
+              k_new.stride(0), k_new.stride(1), v_new.stride(0), v_new.stride(1),
+              k_pool.data_ptr(), v_pool.data_ptr(), slot_mapping.data_ptr(),
+              n_tok, hkv, head_dim, bs, num_pages, dtype_code(k_pool.dtype), _stream(dev))
 
 
 def kv_gather(k_pool: torch.Tensor, v_pool: torch.Tensor, block_tables: torch.Tensor,
@@ -241,9 +235,9 @@ def kv_gather(k_pool: torch.Tensor, v_pool: torch.Tensor, block_tables: torch.Te
             if tuple(t.shape) != shape or t.dtype != k_pool.dtype or not t.is_contiguous():
                 raise ValueError(f"gather outputs must be contiguous {shape} {k_pool.dtype}")
             _buffer(t, dev, "gather output")
-    _launch(dev, "ivakv_gather", k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),
-            context_lens.data_ptr(), batch, max_blocks, hkv, head_dim, bs, num_pages, out_len,
-            k_out.data_ptr(), v_out.data_ptr(), dtype_code(k_pool.dtype))
+    _abi.call("ivakv_gather", k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),
+              context_lens.data_ptr(), batch, max_blocks, hkv, head_dim, bs, num_pages, out_len,
+              k_out.data_ptr(), v_out.data_ptr(), dtype_code(k_pool.dtype), _stream(dev))
     return k_out, v_out
 
 
@@ -380,17 +374,18 @@ def _decode(entry: str, q, k_pool, v_pool, block_tables, context_lens, scale, wi
                              f"{nbytes} needed")
         _buffer(workspace, dev, "workspace")
     if scales is not None:
-        _launch(dev, entry, q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),
-                scales[0].data_ptr(), scales[1].data_ptr(), block_tables.data_ptr(),
-                context_lens.data_ptr(), out.data_ptr(), workspace.data_ptr(),
-                workspace.numel() * workspace.element_size(), batch, hq, hkv, head_dim, bs,
-                max_blocks, num_pages, float(scale), window, n_sink, dtype_code(q.dtype))
+        _abi.call(entry, q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),
+                  scales[0].data_ptr(), scales[1].data_ptr(), block_tables.data_ptr(),
+                  context_lens.data_ptr(), out.data_ptr(), workspace.data_ptr(),
+                  workspace.numel() * workspace.element_size(), batch, hq, hkv, head_dim, bs,
+                  max_blocks, num_pages, float(scale), window, n_sink, dtype_code(q.dtype),
+                  _stream(dev))
         return out
-    _launch(dev, entry, q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),
-            context_lens.data_ptr(), out.data_ptr(), workspace.data_ptr(),
-            workspace.numel() * workspace.element_size(), batch, hq, hkv, head_dim, bs,
-            max_blocks, num_pages, float(scale), window, n_sink, partition_pages,
-            dtype_code(q.dtype))
+    _abi.call(entry, q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),
+              context_lens.data_ptr(), out.data_ptr(), workspace.data_ptr(),
+              workspace.numel() * workspace.element_size(), batch, hq, hkv, head_dim, bs,
+              max_blocks, num_pages, float(scale), window, n_sink, partition_pages,
+              dtype_code(q.dtype), _stream(dev))
     return out
 
 
@@ -501,18 +496,20 @@ def paged_decode_append_attention(q: torch.Tensor, k_new: torch.Tensor, v_new: t
                              f"{nbytes} needed")
         _buffer(workspace, dev, "workspace")
     if fp8:
-        _launch(dev, "ivakv_decode_append_attn_fp8", q.data_ptr(), k_new.data_ptr(),
-                v_new.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), scales[0].data_ptr(),
-                scales[1].data_ptr(), block_tables.data_ptr(), context_lens.data_ptr(),
-                out.data_ptr(), workspace.data_ptr(),
-                workspace.numel() * workspace.element_size(), batch, hq, hkv, head_dim, bs,
-                max_blocks, num_pages, float(scale), window, n_sink, dtype_code(q.dtype))
+        _abi.call("ivakv_decode_append_attn_fp8", q.data_ptr(), k_new.data_ptr(),
+                  v_new.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), scales[0].data_ptr(),
+                  scales[1].data_ptr(), block_tables.data_ptr(), context_lens.data_ptr(),
+                  out.data_ptr(), workspace.data_ptr(),
+                  workspace.numel() * workspace.element_size(), batch, hq, hkv, head_dim, bs,
+                  max_blocks, num_pages, float(scale), window, n_sink, dtype_code(q.dtype),
+                  _stream(dev))
         return out
-    _launch(dev, "ivakv_decode_append_attn", q.data_ptr(), k_new.data_ptr(), v_new.data_ptr(),
-            k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),
-            context_lens.data_ptr(), out.data_ptr(), workspace.data_ptr(),
-            workspace.numel() * workspace.element_size(), batch, hq, hkv, head_dim, bs,
-            max_blocks, num_pages, float(scale), window, n_sink, dtype_code(q.dtype))
+    _abi.call("ivakv_decode_append_attn", q.data_ptr(), k_new.data_ptr(), v_new.data_ptr(),
+              k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),
+              context_lens.data_ptr(), out.data_ptr(), workspace.data_ptr(),
+              workspace.numel() * workspace.element_size(), batch, hq, hkv, head_dim, bs,
+              max_blocks, num_pages, float(scale), window, n_sink, dtype_code(q.dtype),
+              _stream(dev))
     return out
 
 
@@ -542,16 +539,16 @@ def _append_fp8(k_new, v_new, k_pool, v_pool, slot_mapping, k_scale, v_scale,
         pos = _i32_row(rope_positions, "rope_positions")
         if pos.numel() != n_tok or pos.device != dev:
             raise ValueError(f"rope_positions must be {n_tok} int32 values on {dev}")
-        _launch(dev, "ivakv_append_rope_fp8", k_new.data_ptr(), v_new.data_ptr(),
-                k_new.stride(0), k_new.stride(1), v_new.stride(0), v_new.stride(1),
-                k_pool.data_ptr(), v_pool.data_ptr(), k_scale.data_ptr(), v_scale.data_ptr(),
-                slot_mapping.data_ptr(), pos.data_ptr(), n_tok, hkv, head_dim, bs, num_pages,
-                float(rope_theta), code)
+        _abi.call("ivakv_append_rope_fp8", k_new.data_ptr(), v_new.data_ptr(),
+                  k_new.stride(0), k_new.stride(1), v_new.stride(0), v_new.stride(1),
+                  k_pool.data_ptr(), v_pool.data_ptr(), k_scale.data_ptr(), v_scale.data_ptr(),
+                  slot_mapping.data_ptr(), pos.data_ptr(), n_tok, hkv, head_dim, bs, num_pages,
+                  float(rope_theta), code, _stream(dev))
         return
-    _launch(dev, "ivakv_append_fp8", k_new.data_ptr(), v_new.data_ptr(),
-            k_new.stride(0), k_new.stride(1), v_new.stride(0), v_new.stride(1),
-            k_pool.data_ptr(), v_pool.data_ptr(), k_scale.data_ptr(), v_scale.data_ptr(),
-            slot_mapping.data_ptr(), n_tok, hkv, head_dim, bs, num_pages, code)
+    _abi.call("ivakv_append_fp8", k_new.data_ptr(), v_new.data_ptr(),
+              k_new.stride(0), k_new.stride(1), v_new.stride(0), v_new.stride(1),
+              k_pool.data_ptr(), v_pool.data_ptr(), k_scale.data_ptr(), v_scale.data_ptr(),
+              slot_mapping.data_ptr(), n_tok, hkv, head_dim, bs, num_pages, code, _stream(dev))
 
 
 def _gather_fp8(k_pool, v_pool, block_tables, context_lens, out_len, out, k_scale, v_scale,
@@ -576,10 +573,10 @@ def _gather_fp8(k_pool, v_pool, block_tables, context_lens, out_len, out, k_scal
             if tuple(t.shape) != shape or not t.is_contiguous() or t.dtype != k_out.dtype:
                 raise ValueError(f"gather outputs must be contiguous {shape}, one dtype")
             _buffer(t, dev, "gather output")
-    _launch(dev, "ivakv_gather_fp8", k_pool.data_ptr(), v_pool.data_ptr(), k_scale.data_ptr(),
-            v_scale.data_ptr(), block_tables.data_ptr(), context_lens.data_ptr(), batch,
-            max_blocks, hkv, head_dim, bs, num_pages, out_len, k_out.data_ptr(),
-            v_out.data_ptr(), dtype_code(k_out.dtype))
+    _abi.call("ivakv_gather_fp8", k_pool.data_ptr(), v_pool.data_ptr(), k_scale.data_ptr(),
+              v_scale.data_ptr(), block_tables.data_ptr(), context_lens.data_ptr(), batch,
+              max_blocks, hkv, head_dim, bs, num_pages, out_len, k_out.data_ptr(),
+              v_out.data_ptr(), dtype_code(k_out.dtype), _stream(dev))
     return k_out, v_out
 
 
@@ -674,30 +671,32 @@ def paged_prefill_attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch
         _buffer(workspace, dev, "workspace")
         ws = (workspace.data_ptr(), workspace.numel() * workspace.element_size())
         if fp8:
-            _launch(dev, "ivakv_prefill_attn_split_fp8", q.data_ptr(), k_pool.data_ptr(),
-                    v_pool.data_ptr(), scales[0].data_ptr(), scales[1].data_ptr(),
-                    block_tables.data_ptr(), context_lens.data_ptr(), query_start.data_ptr(),
-                    q.shape[0], out.data_ptr(), *ws, batch, hq, hkv, head_dim, bs, max_blocks,
-                    num_pages, int(max_query_len), float(scale), window, n_sink,
-                    dtype_code(q.dtype))
+            _abi.call("ivakv_prefill_attn_split_fp8", q.data_ptr(), k_pool.data_ptr(),
+                      v_pool.data_ptr(), scales[0].data_ptr(), scales[1].data_ptr(),
+                      block_tables.data_ptr(), context_lens.data_ptr(), query_start.data_ptr(),
+                      q.shape[0], out.data_ptr(), *ws, batch, hq, hkv, head_dim, bs, max_blocks,
+                      num_pages, int(max_query_len), float(scale), window, n_sink,
+                      dtype_code(q.dtype), _stream(dev))
         else:
-            _launch(dev, "ivakv_prefill_attn_split", q.data_ptr(), k_pool.data_ptr(),
-                    v_pool.data_ptr(), block_tables.data_ptr(), context_lens.data_ptr(),
-                    query_start.data_ptr(), q.shape[0], out.data_ptr(), *ws, batch, hq, hkv,
-                    head_dim, bs, max_blocks, num_pages, int(max_query_len), float(scale),
-                    window, n_sink, dtype_code(q.dtype))
+            _abi.call("ivakv_prefill_attn_split", q.data_ptr(), k_pool.data_ptr(),
+                      v_pool.data_ptr(), block_tables.data_ptr(), context_lens.data_ptr(),
+                      query_start.data_ptr(), q.shape[0], out.data_ptr(), *ws, batch, hq, hkv,
+                      head_dim, bs, max_blocks, num_pages, int(max_query_len), float(scale),
+                      window, n_sink, dtype_code(q.dtype), _stream(dev))
         return out
     if fp8:
-        _launch(dev, "ivakv_prefill_attn_fp8", q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),
-                scales[0].data_ptr(), scales[1].data_ptr(), block_tables.data_ptr(),
-                context_lens.data_ptr(), query_start.data_ptr(), q.shape[0], out.data_ptr(),
-                batch, hq, hkv, head_dim, bs, block_tables.shape[1], num_pages,
-                int(max_query_len), float(scale), window, n_sink, dtype_code(q.dtype))
+        _abi.call("ivakv_prefill_attn_fp8", q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),
+                  scales[0].data_ptr(), scales[1].data_ptr(), block_tables.data_ptr(),
+                  context_lens.data_ptr(), query_start.data_ptr(), q.shape[0], out.data_ptr(),
+                  batch, hq, hkv, head_dim, bs, block_tables.shape[1], num_pages,
+                  int(max_query_len), float(scale), window, n_sink, dtype_code(q.dtype),
+                  _stream(dev))
         return out
-    _launch(dev, "ivakv_prefill_attn", q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),
-            block_tables.data_ptr(), context_lens.data_ptr(), query_start.data_ptr(),
-            q.shape[0], out.data_ptr(), batch, hq, hkv, head_dim, bs, block_tables.shape[1],
-            num_pages, int(max_query_len), float(scale), window, n_sink, dtype_code(q.dtype))
+    _abi.call("ivakv_prefill_attn", q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),
+              block_tables.data_ptr(), context_lens.data_ptr(), query_start.data_ptr(),
+              q.shape[0], out.data_ptr(), batch, hq, hkv, head_dim, bs, block_tables.shape[1],
+              num_pages, int(max_query_len), float(scale), window, n_sink, dtype_code(q.dtype),
+              _stream(dev))
     return out
 
 
@@ -712,8 +711,8 @@ def rope_(x: torch.Tensor, positions: torch.Tensor, theta: float = 10000.0) -> t
     pos = _i32(positions, "positions").reshape(-1)
     if pos.numel() != x.shape[0]:
         raise ValueError(f"{pos.numel()} positions for {x.shape[0]} rows")
-    _launch(dev, "ivakv_rope", x.data_ptr(), x.stride(0), x.stride(1), pos.data_ptr(), x.shape[0],
-            x.shape[1], x.shape[2], float(theta), dtype_code(x.dtype))
+    _abi.call("ivakv_rope", x.data_ptr(), x.stride(0), x.stride(1), pos.data_ptr(), x.shape[0],
+              x.shape[1], x.shape[2], float(theta), dtype_code(x.dtype), _stream(dev))
     return x
 
 
@@ -729,8 +728,8 @@ def chunk_slots(block_tables: torch.Tensor, context_lens: torch.Tensor, n: int,
     if block_tables.dim() != 2 or block_tables.shape[0] != batch:
         raise ValueError("block_tables must be [B, max_blocks] with B == len(context_lens)")
     out = torch.empty(batch * n, dtype=torch.int32, device=dev)
-    _launch(dev, "ivakv_chunk_slots", block_tables.data_ptr(), context_lens.data_ptr(), batch, n,
-            block_tables.shape[1], block_size, out.data_ptr())
+    _abi.call("ivakv_chunk_slots", block_tables.data_ptr(), context_lens.data_ptr(), batch, n,
+              block_tables.shape[1], block_size, out.data_ptr(), _stream(dev))
     return out
 
 
@@ -749,19 +748,18 @@ def rms_norm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float,
     out = torch.empty_like(x)
     total = torch.empty_like(x) if residual is not None else None
     d = x.shape[-1]
-    _launch(x.device, "ivakv_rms_norm", x.data_ptr(),
-            residual.data_ptr() if residual is not None else None,
-            weight.data_ptr() if weight is not None else None,
-            total.data_ptr() if total is not None else None, out.data_ptr(), x.numel() // d, d,
-            eps, dtype_code(x.dtype))
+    _abi.call("ivakv_rms_norm", x.data_ptr(), residual.data_ptr() if residual is not None else None,
+              weight.data_ptr() if weight is not None else None,
+              total.data_ptr() if total is not None else None, out.data_ptr(), x.numel() // d, d,
+              eps, dtype_code(x.dtype), _stream(x.device))
     return out if total is None else (total, out)
 
 
 def swiglu(up: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """silu(up) * gate (src/core/ffn.py:21-24,57-60)."""
     out = torch.empty_like(up)
-    _launch(up.device, "ivakv_swiglu", up.data_ptr(), gate.data_ptr(), out.data_ptr(), up.numel(),
-            dtype_code(up.dtype))
+    _abi.call("ivakv_swiglu", up.data_ptr(), gate.data_ptr(), out.data_ptr(), up.numel(),
+              dtype_code(up.dtype), _stream(up.device))
     return out
 
 
@@ -789,9 +787,10 @@ def linear_rows(x: torch.Tensor, weights, norm=None, residual: Optional[torch.Te
         norm3 = _NO_NORM
     else:
         norm3 = (1, norm[0].data_ptr() if norm[0] is not None else None, norm[1])
-    _launch(x.device, "ivakv_linear_rows", x.data_ptr(), k, x.numel() // k, k, *args,
-            residual.data_ptr() if residual is not None else None, *norm3,
-            2 if swiglu_pair else 1 if residual is not None else 0, dtype_code(x.dtype))
+    _abi.call("ivakv_linear_rows", x.data_ptr(), k, x.numel() // k, k, *args,
+              residual.data_ptr() if residual is not None else None, *norm3,
+              2 if swiglu_pair else 1 if residual is not None else 0, dtype_code(x.dtype),
+              _stream(x.device))
     return outs if len(outs) > 1 else outs[0]
 
 
@@ -822,7 +821,7 @@ def block_decode(x: torch.Tensor, norm1, eps1: float, wq, wk, wv, wo, norm2, eps
         context_lens.data_ptr(), scratch.data_ptr(), nbytes, ws.data_ptr(), ws.numel(), m, d, num_q_heads,
         hkv, head_dim, hidden, bs, max_blocks, num_pages, window, n_sink, dtype_code(x.dtype), int(fp8),
         eps1, eps2, scale)
-    _launch(dev, "ivakv_block_decode", args)
+    _abi.call("ivakv_block_decode", args, _stream(dev))
     return out
 
 
@@ -849,11 +848,11 @@ def copy_pages(k_pool: torch.Tensor, v_pool: torch.Tensor, src_pages: torch.Tens
         ks, vs = _scales(k_pool, k_scale, v_scale)
     for start in range(0, src.numel(), 65535):
         n = min(65535, src.numel() - start)
-        _launch(dev, "ivakv_copy_pages", k_pool.data_ptr(), v_pool.data_ptr(),
-                ks.data_ptr() if ks is not None else None,
-                vs.data_ptr() if vs is not None else None,
-                src[start:].data_ptr(), dst[start:].data_ptr(), n, num_pages, hkv, head_dim,
-                bs, k_pool.element_size())
+        _abi.call("ivakv_copy_pages", k_pool.data_ptr(), v_pool.data_ptr(),
+                  ks.data_ptr() if ks is not None else None,
+                  vs.data_ptr() if vs is not None else None,
+                  src[start:].data_ptr(), dst[start:].data_ptr(), n, num_pages, hkv, head_dim,
+                  bs, k_pool.element_size(), _stream(dev))
 
 
 def kv_compact(kv_cache: torch.Tensor, mask: torch.Tensor) -> torch.Tensor:
@@ -928,14 +927,15 @@ def _kv_ops(kv_cache: torch.Tensor, indices: torch.Tensor, values: Optional[torc
     code = dtype_code(kv_cache.dtype)
     if operation == "gather":
         out = torch.empty((batch, n_heads, n_idx, head_dim), dtype=kv_cache.dtype, device=dev)
-        _launch(dev, "ivakv_index_gather", kv_cache.data_ptr(), *kv_cache.stride(), idx.data_ptr(),
-                n_idx, batch, n_heads, seq_len, head_dim, out.data_ptr(), code)
+        _abi.call("ivakv_index_gather", kv_cache.data_ptr(), *kv_cache.stride(), idx.data_ptr(),
+                  n_idx, batch, n_heads, seq_len, head_dim, out.data_ptr(), code, _stream(dev))
         return out
     if tuple(values.shape) != (batch, n_heads, n_idx, head_dim):
         raise ValueError(f"values must be {(batch, n_heads, n_idx, head_dim)}; got {tuple(values.shape)}")
     if values.dtype != kv_cache.dtype:
         raise TypeError(f"values dtype {values.dtype} != cache dtype {kv_cache.dtype}")
     out = kv_cache.clone()
-    _launch(dev, "ivakv_index_scatter", out.data_ptr(), *out.stride(), idx.data_ptr(), n_idx,
-            values.data_ptr(), *values.stride(), batch, n_heads, seq_len, head_dim, code)
+    _abi.call("ivakv_index_scatter", out.data_ptr(), *out.stride(), idx.data_ptr(), n_idx,
+              values.data_ptr(), *values.stride(), batch, n_heads, seq_len, head_dim, code,
+              _stream(dev))
     return out

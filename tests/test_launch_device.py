@@ -68,7 +68,8 @@ def test_launch_enters_the_tensors_device(iva, monkeypatch, entry, current):
     monkeypatch.setattr(ops, "_raw_stream", lambda index: 100 + index)
     monkeypatch.setattr(torch, "empty", lambda *a, **k: _OnGpu1(4))
     monkeypatch.setattr(torch, "empty_like", lambda t: t)
-    monkeypatch.setattr(ops._abi, "call", lambda name, *a: seen.append((name, state["current"], a[-1])))
+    monkeypatch.setitem(ops._abi._FUNCS, entry,
+                        lambda *a: seen.append((entry, state["current"], a[-1])) or ops._abi.OK)
     CALLS[entry](ops, _OnGpu1)
     assert seen == [(entry, 1, 101)]
     assert state["current"] == current
