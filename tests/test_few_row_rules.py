@@ -1,6 +1,6 @@
-"""Where the few-row linear kernel is taken: by rows and widths, and not where its loss to the
+"""Where the layer kernels are taken.  The few-row linear kernel: by rows and widths, and not where its loss to the
 library's products on the GPU outgrows what its fewer calls save the host.  The modules run on the meta device with the kernels stood
-in, so that wide ones cost nothing."""
+in, so that wide ones cost nothing.  RMSNorm's kernel: not for many very narrow rows."""
 from __future__ import annotations
 
 import pytest
@@ -85,3 +85,16 @@ def test_head(iva, taken, d, vocab, rows, kernel):
         head.token_embedding, head.lm_head = torch.nn.Embedding(vocab, d), None
     assert head.logits(_x(rows, d)).shape == (rows, 1, vocab)
     assert taken == [[rows, d, vocab]] * kernel
+
+
+@pytest.mark.parametrize("d,rows,kernel", [
+    (8, 1 << 16, True), (8, (1 << 16) + 1, False), (24, 1 << 16, True), (24, 1 << 20, False),
+    (32, 1 << 20, True), (4096, 1 << 20, True)])
+def test_norm_of_many_narrow_rows_leaves_the_kernel(iva, taken, monkeypatch, d, rows, kernel):
+    M, norms = iva.model, []
+    monkeypatch.setattr(M, "rms_norm", lambda x, w, eps: norms.append(tuple(x.shape)) or x)
+    cfg = iva.TransformerConfig(d_model=d, n_heads=1, n_kv_heads=1, n_layers=1, vocab_size=64, seq_len=8, dropout=0.0)
+    with torch.device("meta"):
+        norm = M.RMSNorm(cfg)
+    norm(_x(rows, d))
+    assert bool(norms) == kernel
